@@ -134,7 +134,11 @@ enum {
                              (STORE, STORE_BIAS, ADD_RESID, SWIGLU_FWD), NT in one pass (STORE, K up
                              to about 4000 rows at m <= 4). PXK_TILE_AUTO picks it whenever it applies */
     PXK_TILE_32x48_DIRECT = 8, /* as 32x64 direct, 48 columns: 192 workgroups over a 512 x 576 output */
-    PXK_TILE_32x48 = 9        /* as 32x64, 48 columns */
+    PXK_TILE_32x48 = 9,       /* as 32x64, 48 columns */
+    /* fp32 products on the bf16 matrix units, every operand split exactly into three bf16 parts
+     * (fp32 accumulation; no less exact than the fp32 MFMA, gemm_impl.hpp) */
+    PXK_TILE_128x128_SPLIT = 10,
+    PXK_TILE_64x64_SPLIT = 11
 };
 
 typedef struct pxk_gemm_desc {
@@ -176,7 +180,11 @@ typedef struct pxk_gemm_desc {
     const float* x_gamma;
     float* row_rms;          /* PXK_PRO_RMS: receives rms[m] (nullable) */
     float norm_eps;          /* PXK_PRO_RMS */
-    int32_t reserved2;
+    int32_t denominator;     /* 1: the product is, or feeds, a denominator of the epsilon rules (a forward
+                                pass kept for a relevance pass): PXK_TILE_AUTO then plans over the fp32
+                                tiles alone, whose rounding those rules' results have always had. Near a
+                                zero denominator eps / z turns a last-bit difference of z into one of the
+                                relevance, whichever of two equally exact products z came from. */
 } pxk_gemm_desc;
 
 /* Bytes of workspace pxk_gemm needs for this descriptor (0 when it runs without split-K). */

@@ -67,6 +67,12 @@ inline pxk_gemm_desc gemm_desc(int64_t m, int64_t n, int64_t k) {
     d.batch = d.inner = d.kgroups = 1;
     return d;
 }
+/** @brief gemm_desc for a forward product that is, or feeds, a denominator of the relevance pass. */
+inline pxk_gemm_desc forward_desc(int64_t m, int64_t n, int64_t k) {
+    pxk_gemm_desc d = gemm_desc(m, n, k);
+    d.denominator = 1;
+    return d;
+}
 
 /** @brief The stabilizer bias a rule puts in a Linear's denominator: the layer's bias under the
  *         bias-in-denominator epsilon rule, none under the pre-bias rule (lrp_rules.cpp:197-220). */

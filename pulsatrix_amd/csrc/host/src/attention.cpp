@@ -175,7 +175,7 @@ const float* MultiHeadAttentionModule::run_forward(const float* x, int64_t n, in
     const bool qkn = config_.use_qk_norm;
     const bool rope_in_gemm = config_.use_rope && !qkn && (w3 <= 128 || 128 % D_ == 0);
     {
-        pxk_gemm_desc d = gemm_desc(l, w3, d_);
+        pxk_gemm_desc d = detail::forward_desc(l, w3, d_);
         d.batch = n;
         d.a = mat(x, d_, l * d_);
         d.b = mat(wqkv_.data(), w3);
@@ -246,7 +246,7 @@ const float* MultiHeadAttentionModule::run_forward(const float* x, int64_t n, in
     float* oz = out_z_.ensure(be_, M * d_);
     float* oy = config_.out_bias ? out_y_.ensure(be_, M * d_) : oz;
     {
-        pxk_gemm_desc d = gemm_desc(M, d_, qd);
+        pxk_gemm_desc d = detail::forward_desc(M, d_, qd);
         d.a = mat(ctx, qd);
         d.b = mat(out_proj_.weight_data(), d_);
         d.c = mat(oz, d_);
@@ -409,7 +409,7 @@ void MultiHeadAttentionModule::run_attention_unfused(const float* q, int64_t ldq
     float* ctx = ctx_.data();
     // 3. raw scores = Q K^T per query head; K read through the KV-head map.
     {
-        pxk_gemm_desc d = gemm_desc(l, l, D_);
+        pxk_gemm_desc d = detail::forward_desc(l, l, D_);
         d.batch = n * H_;
         d.inner = H_;
         d.trans_b = 1;
@@ -424,7 +424,7 @@ void MultiHeadAttentionModule::run_attention_unfused(const float* q, int64_t ldq
                          "MultiHeadAttentionModule::forward (softmax)");
     // 5. context = P V, written head-packed (N*L, H*D): the merge permute is the store layout.
     {
-        pxk_gemm_desc d = gemm_desc(l, D_, l);
+        pxk_gemm_desc d = detail::forward_desc(l, D_, l);
         d.batch = n * H_;
         d.inner = H_;
         d.causal = causal ? PXK_CAUSAL_K_LE_M : PXK_CAUSAL_NONE;

@@ -85,7 +85,7 @@ const float* SwiGLUModule::run_forward(const float* x, int64_t rows, const float
     float* gp = gate_post_.ensure(be_, rows * F_);
     float* h = hidden_.ensure(be_, rows * F_);
     if (fused_gate()) {  // gate and up projections and the gate itself in one GEMM
-        pxk_gemm_desc d = gemm_desc(rows, f2, d_);
+        pxk_gemm_desc d = detail::forward_desc(rows, f2, d_);
         d.a = mat(x, d_);
         d.b = mat(wgu_il_.data(), f2);
         d.c = mat(gz, f2);
@@ -96,7 +96,7 @@ const float* SwiGLUModule::run_forward(const float* x, int64_t rows, const float
         fold(d);
         be_->run_gemm(d);
     } else {  // gate and up projections in one GEMM, then the gate
-        pxk_gemm_desc d = gemm_desc(rows, f2, d_);
+        pxk_gemm_desc d = detail::forward_desc(rows, f2, d_);
         d.a = mat(x, d_);
         d.b = mat(wgu_.data(), f2);
         d.c = mat(gz, f2);
@@ -113,7 +113,7 @@ const float* SwiGLUModule::run_forward(const float* x, int64_t rows, const float
     float* dz = down_z_.ensure(be_, rows * d_);
     float* dy = use_bias_ ? down_y_.ensure(be_, rows * d_) : dz;
     {
-        pxk_gemm_desc d = gemm_desc(rows, d_, F_);
+        pxk_gemm_desc d = detail::forward_desc(rows, d_, F_);
         d.a = mat(h, F_);
         d.b = mat(down_proj_.weight_data(), d_);
         d.c = mat(dz, d_);

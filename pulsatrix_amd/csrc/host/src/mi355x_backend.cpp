@@ -190,9 +190,10 @@ void MI355XBackend::run_gemm(pxk_gemm_desc& d) {
         int32_t tile = 0, splits = 0;
         check(pxk_gemm_plan(&d, &tile, &splits), "MI355XBackend gemm (plan)");
         static const char* const kTile[] = {"auto",   "128x128", "64x64",  "32x64",  "32x32",
-                                            "32x64d", "32x32d",  "skinny", "32x48d", "32x48"};
+                                            "32x64d", "32x32d",  "skinny", "32x48d", "32x48",
+                                            "128x128s", "64x64s"};
         char name[96];
-        std::snprintf(name, sizeof(name), "gemm %s %s%s pro%d epi%d split%d", kTile[tile >= 0 && tile <= 9 ? tile : 0],
+        std::snprintf(name, sizeof(name), "gemm %s %s%s pro%d epi%d split%d", kTile[tile >= 0 && tile <= 11 ? tile : 0],
                       d.trans_a ? "T" : "N", d.trans_b ? "T" : "N", d.prologue, d.epilogue, splits);
         // Algorithmic bytes: every operand once (A, B, the prologue's denominators, the
         // epilogue's inputs and outputs), none of the split-K partials or re-reads.
@@ -275,6 +276,7 @@ void MI355XBackend::gemm_ex(const float* a, bool ta, const float* b, bool tb, fl
                             size_t n, float beta) {
     if (m == 0 || n == 0) return;
     pxk_gemm_desc d{};
+    d.denominator = 1;  // a module's forward may be kept for its relevance pass
     d.m = static_cast<int64_t>(m);
     d.n = static_cast<int64_t>(n);
     d.k = static_cast<int64_t>(k);
@@ -294,6 +296,7 @@ void MI355XBackend::gemm_strided_batched(const float* a, bool ta, size_t stride_
                                          size_t batch, float beta) {
     if (m == 0 || n == 0 || batch == 0) return;
     pxk_gemm_desc d{};
+    d.denominator = 1;  // a module's forward may be kept for its relevance pass
     d.m = static_cast<int64_t>(m);
     d.n = static_cast<int64_t>(n);
     d.k = static_cast<int64_t>(k);

@@ -68,7 +68,7 @@ const float* LinearModule::run_forward(const float* x, int64_t rows) {
     x_ = x;
     rows_ = rows;
     float* z = z_.ensure(be_, rows * out_);
-    pxk_gemm_desc d = gemm_desc(rows, out_, in_);
+    pxk_gemm_desc d = detail::forward_desc(rows, out_, in_);
     d.a = mat(x, in_);
     d.b = mat(weight_.data(), out_);
     d.c = mat(z, out_);

@@ -11,44 +11,40 @@ const Table kTables[] = {{kTable0, kTable0Size}, {kTable1, kTable1Size}, {kTable
 
 // Plan index <-> PXK_TILE_*: the MFMA tiles in table order, the skinny kernels after them.
 constexpr int kSkinnyTile = kTiles;
-int public_tile(int t) {
-    if (t < 6) return t + 1;
-    if (t == 6) return PXK_TILE_32x48_DIRECT;
-    return t == 7 ? PXK_TILE_32x48 : PXK_TILE_SKINNY;
-}
+constexpr int kPublicTile[kTiles] = {PXK_TILE_128x128, PXK_TILE_64x64, PXK_TILE_32x64, PXK_TILE_32x32,
+                                     PXK_TILE_32x64_DIRECT, PXK_TILE_32x32_DIRECT, PXK_TILE_32x48_DIRECT, PXK_TILE_32x48,
+                                     PXK_TILE_128x128_SPLIT, PXK_TILE_64x64_SPLIT};
+int public_tile(int t) { return t < kTiles ? kPublicTile[t] : PXK_TILE_SKINNY; }
 int plan_tile(int id) {  // -1: none
-    if (id >= PXK_TILE_128x128 && id <= PXK_TILE_32x32_DIRECT) return id - 1;
-    if (id == PXK_TILE_32x48_DIRECT) return 6;
-    if (id == PXK_TILE_32x48) return 7;
+    for (int t = 0; t < kTiles; ++t)
+        if (kPublicTile[t] == id) return t;
     return id == PXK_TILE_SKINNY ? kSkinnyTile : -1;
 }
 
 struct TileInfo {
-    int bm, bn, bk, threads, smem_bytes;
+    int bm, bn, bk, threads;
     double floor_us;  // a K stage of a workgroup alone on its CU (load latency bound), measured
-    double util;      // MFMA utilisation when several waves share a SIMD, measured
+    double util;      // fp32 MFMA utilisation when several waves share a SIMD, measured (the split
+                      // tiles' products run on the bf16 units: above 1)
     bool direct;      // waves stream their operands from L2 into registers (no LDS panels)
+    bool whole;       // fast on whole tiles of aligned operands only (element-wise guards elsewhere)
 };
 
-template <class C>
-constexpr int smem_of() {
-    // The largest of the four (TA, TB) layouts: what a CU must hold for one workgroup.
-    int s = Layout<C, false, false>::SIZE;
-    if (Layout<C, false, true>::SIZE > s) s = Layout<C, false, true>::SIZE;
-    if (Layout<C, true, false>::SIZE > s) s = Layout<C, true, false>::SIZE;
-    if (Layout<C, true, true>::SIZE > s) s = Layout<C, true, true>::SIZE;
-    return 4 * s;
-}
-
+// The split tiles' figures: 8192 x 2048 x 2048 gives 1.4 us per stage and workgroup of a CU for
+// 128x128 and 3072 x 3072 x 576 0.47 for 64x64 (0.54 at three to a CU: 512 x 576 x 3072 in 8 splits);
+// a lone workgroup (512 x 576 x 1536) 1.8 and 0.65.
+constexpr int kFp32Tiles = 8;
 const TileInfo kTileInfo[kTiles] = {
-    {128, 128, 32, C128::NT, smem_of<C128>(), 1.0, 0.75, false},
-    {64, 64, 32, C64::NT, smem_of<C64>(), 0.8, 0.65, false},
-    {32, 64, 64, C32x64::NT, smem_of<C32x64>(), 0.8, 0.55, false},
-    {32, 32, 64, C32::NT, smem_of<C32>(), 0.8, 0.5, false},
-    {32, 64, 64, C32x64::NT, 4 * C32x64::KS * 32 * C32x64::LDC, 0.65, 0.55, true},
-    {32, 32, 64, C32::NT, 4 * C32::KS * 32 * C32::LDC, 0.65, 0.5, true},
-    {32, 48, 64, C32x48::NT, 4 * C32x48::KS * 32 * C32x48::LDC, 0.65, 0.55, true},
-    {32, 48, 64, C32x48::NT, smem_of<C32x48>(), 0.8, 0.55, false},
+    {128, 128, 32, C128::NT, 1.0, 0.75, false, true},
+    {64, 64, 32, C64::NT, 0.8, 0.65, false, true},
+    {32, 64, 64, C32x64::NT, 0.8, 0.55, false, true},
+    {32, 32, 64, C32::NT, 0.8, 0.5, false, true},
+    {32, 64, 64, C32x64::NT, 0.65, 0.55, true, false},
+    {32, 32, 64, C32::NT, 0.65, 0.5, true, false},
+    {32, 48, 64, C32x48::NT, 0.65, 0.55, true, false},
+    {32, 48, 64, C32x48::NT, 0.8, 0.55, false, true},
+    {128, 128, 32, S128::NT, 1.8, 1.18, false, false},
+    {64, 64, 32, S64::NT, 0.65, 0.79, false, false},
 };
 
 constexpr int kSkinnyMaxLds = 64 * 1024;
@@ -95,6 +91,13 @@ bool vec_ok(const pxk_operand& o, int64_t contiguous_extent) {
     return aligned16(o.ptr) && o.ld % 4 == 0 && o.batch_stride % 4 == 0 && o.inner_stride % 4 == 0 &&
            o.group_stride % 4 == 0 && contiguous_extent % 4 == 0;
 }
+
+// 16-byte aligned rows of A (and the prologue's operands) and of B.
+bool vec_a(const pxk_gemm_desc* d) {
+    const int64_t ext = d->trans_a ? d->m : d->k;
+    return vec_ok(d->a, ext) && (d->prologue == PXK_PRO_NONE || (vec_ok(d->z, ext) && vec_ok(d->z_bias, ext)));
+}
+bool vec_b(const pxk_gemm_desc* d) { return vec_ok(d->b, d->trans_b ? d->k : d->n); }
 
 struct Plan {
     const Entry* e;
@@ -153,9 +156,10 @@ double estimate(const pxk_gemm_desc* d, const TileInfo& t, double tiles, double 
         // tiles run 10-25% slower than from LDS panels (measured; without the prologue they win).
         floor = 1.0;
         util *= 0.65;
-    } else if (t.direct && d->trans_b && waves_per_simd > 1.0) {
+    } else if (t.direct && (d->trans_b || !d->denominator) && waves_per_simd > 1.0) {
         // The same fragment-shaped loads with two or more workgroups per CU: they saturate the
-        // vector memory path (a 512 x 1536 x 576 NT product runs 1.2-1.9 us faster on LDS panels).
+        // vector memory path (a 512 x 1536 x 576 NT product runs 1.2-1.9 us faster on LDS panels, a
+        // 2048 x 576 x 1536 NN one 59 us on 32x48 direct, 45 on LDS panels and 40 on 64x64 split).
         util *= 0.75;
     }
     const double stage_us = std::max(floor, waves_per_simd * mfma_us / util);
@@ -283,6 +287,7 @@ int plan(const pxk_gemm_desc* d, Plan* p) {
     p->kc = 0;
 
     // Tile shape and split count: the forced ones, else the cheapest by estimate().
+    const bool aligned = vec_a(d) && vec_b(d);
     int best_t = -1, best_s = 1;
     double best = 0.0;
     for (int t = 0; t < kTiles; ++t) {
@@ -292,16 +297,26 @@ int plan(const pxk_gemm_desc* d, Plan* p) {
         if (epi == PXK_EPI_SWIGLU_FWD && ti.bn % 64 != 0) continue;
         const double stages = max_stages(d, ti.bm, ti.bk);
         const double tiles = static_cast<double>(live_tiles(d, ti.bm, ti.bn));
-        // The 128x128 tile only pays off when its tiles alone fill the chip, unless it is the only
-        // one that holds whole heads for a RoPE epilogue.
+        // The 128x128 fp32 tile only pays off when its tiles alone fill the chip, unless it is the only
+        // fp32 one that holds whole heads for a RoPE epilogue.
         const bool rope_epi = epi == PXK_EPI_ROPE_REL || epi == PXK_EPI_ROPE_FWD;
         const bool big_only = d->tile == 0 && t == 0 && !(rope_epi && !rope_fits(d, 64));
         if (big_only && tiles < 256.0) continue;
+        if (d->tile == 0 && !d->denominator) {
+            // The split tiles stand in the place of the fp32 ones of their size.
+            if (t < 2) continue;
+            // A tile that guards element by element whatever touches an edge (512 x 577 x 1531: 2-3x
+            // the time) is left to shapes without edges; the split and direct tiles clamp instead.
+            if (ti.whole && !(aligned && d->m % ti.bm == 0 && d->n % ti.bn == 0 && d->k % ti.bk == 0)) continue;
+        }
+        if (d->tile == 0 && d->denominator && t >= kFp32Tiles) continue;
         for (int s = 1; s <= 64; s *= 2) {
             if (d->splits > 0 && s != 1) break;
             if (d->prologue == PXK_PRO_RMS && s != 1) break;  // the rows' sums of squares need the whole K
             const int splits = d->splits > 0 ? d->splits : s;
             if (d->splits == 0 && s > 1 && (big_only || stages / s < 2.0)) break;
+            // A split of the library's own choice fits pxk_gemm_noalloc's scratch.
+            if (d->splits == 0 && !d->denominator && s > 1 && 4.0 * s * d->batch * d->m * d->n > PXK_GEMM_SCRATCH_BYTES) break;
             const double us = estimate(d, ti, tiles, stages, splits);
             if (best_t < 0 || us < best) {
                 best = us;
@@ -420,17 +435,10 @@ extern "C" int pxk_gemm(const pxk_gemm_desc* d, void* stream) {
     g.rope_cols = d->rope_cols;
     g.gate_act = d->gate_act;
     g.ws = d->workspace;
-    // 128-bit loads when every base, stride and the contiguous extent allow them; the causal
-    // K ranges start at multiples of the tile height, so they keep the alignment.
-    const int64_t a_ext = d->trans_a ? d->m : d->k, b_ext = d->trans_b ? d->k : d->n;
-    g.vec_a = vec_ok(d->a, a_ext) && (d->prologue == PXK_PRO_NONE || (vec_ok(d->z, a_ext) && vec_ok(d->z_bias, a_ext)));
-    g.vec_b = vec_ok(d->b, b_ext);
-    g.vec_e = d->n % 4 == 0 && vec_ok(d->c, d->n) && vec_ok(d->c2, d->n) && vec_ok(d->c3, d->n) &&
-              vec_ok(d->x, d->n) && vec_ok(d->y, d->n) && vec_ok(d->w, d->n) && vec_ok(d->z2, d->n) &&
-              vec_ok(d->z3, d->n) && vec_ok(d->e_bias, d->n) && vec_ok(d->e_bias2, d->n) &&
-              vec_ok(d->c2_den, d->n) && vec_ok(d->c2_den_bias, d->n) &&
-              (d->x_gamma == nullptr || aligned16(d->x_gamma)) &&
-              (d->epilogue == PXK_EPI_ROPE_REL || d->epilogue == PXK_EPI_VALUE_REL ? vec_ok(d->z, d->n) : true);
+    // The causal K ranges start at multiples of the tile height, so they keep the alignment.
+    g.vec_a = vec_a(d);
+    g.vec_b = vec_b(d);
+    g.vec_e = d->n % 4 == 0;
     g.tiles_m = static_cast<int>(p.tiles_m);
     g.tiles_n = static_cast<int>(p.tiles_n);
     g.kc = p.kc;
@@ -455,8 +463,10 @@ extern "C" int pxk_gemm(const pxk_gemm_desc* d, void* stream) {
     g.group_m = g.remap ? group_m(p.tiles_m, p.tiles_n, blocks / 8, kTileInfo[p.tile].bm, kTileInfo[p.tile].bn)
                         : g.tiles_m;
     const int has_bias = d->prologue == PXK_PRO_DIV_STAB && d->z_bias.ptr != nullptr;
-    PXK_LAUNCH(p.e->k[has_bias][p.tile], dim3(static_cast<unsigned>(blocks)),
-                       dim3(static_cast<unsigned>(kTileInfo[p.tile].threads)), 0, S(stream), g);
+    const TileInfo& ti = kTileInfo[p.tile];
+    const bool edges = ti.direct && (d->m % ti.bm != 0 || d->n % ti.bn != 0 || d->k % 16 != 0);
+    const KernelFn kernel = edges ? p.e->edge[has_bias][p.tile - kDirect] : p.e->k[has_bias][p.tile];
+    PXK_LAUNCH(kernel, dim3(static_cast<unsigned>(blocks)), dim3(static_cast<unsigned>(ti.threads)), 0, S(stream), g);
     if (const int rc = launched("pxk_gemm")) return rc;
     if (p.splits > 1) {
         const int bn = kTileInfo[p.tile].bn;

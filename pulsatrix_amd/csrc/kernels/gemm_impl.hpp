@@ -47,6 +47,8 @@ namespace pxk {
 namespace gemm {  // shared by every GEMM translation unit
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+// A float4 in memory at any float's address: gfx950 loads and stores 128 bits at dword alignment.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
 struct Op {
     const float* p;
@@ -67,7 +69,8 @@ struct Args {
     const float* sin_t;
     int64_t head_dim, rope_cols;
     int rope_half, gate_act;
-    int vec_a, vec_b, vec_e;  // 128-bit global access allowed: A (and Z), B, epilogue operands
+    int vec_a, vec_b;  // 16-byte aligned rows: A (and Z), B
+    int vec_e;         // whole float4 columns: N a multiple of 4
     int tiles_m, tiles_n, bm;
     int remap;    // XCD-grouped block order
     int group_m;  // M-tiles per group of the tile order (divides tiles_m; tiles_m: M fastest)
@@ -77,7 +80,8 @@ struct Args {
 
 using KernelFn = void (*)(const Args);
 
-constexpr int kTiles = 8;  // PXK_TILE_128x128 .. PXK_TILE_32x32_DIRECT, PXK_TILE_32x48_DIRECT, PXK_TILE_32x48
+constexpr int kDirect = 4, kDirectTiles = 3;
+constexpr int kTiles = 10;  // gemm.hip's kPublicTile names them
 
 // One (transpose, prologue, epilogue) combination: its kernel on every tile shape, without and
 // with a prologue bias over k, and the split-K reduce for each tile width.
@@ -85,6 +89,7 @@ struct Entry {
     int ta, tb, pro, epi;
     KernelFn k[2][kTiles];  // [prologue bias over k present][tile]
     KernelFn r[kTiles];
+    KernelFn edge[2][kDirectTiles];  // the direct tiles' kernels (from kDirect on) for ragged launches
 };
 
 // The skinny kernels built: B layout, epilogue, kernels for up to 4, 8 and 16 rows (NN: with 64-,
@@ -206,7 +211,7 @@ struct Layout {
 
 // ---- 128-bit epilogue access with a scalar tail ------------------------------------------------------
 __device__ __forceinline__ f4 ld4(const float* p, bool vec, int cnt) {
-    if (vec) return *reinterpret_cast<const f4*>(p);
+    if (vec) return *reinterpret_cast<const f4u*>(p);
     f4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -218,7 +223,7 @@ __device__ __forceinline__ f4 ld4(const float* p, bool vec, int cnt) {
 // kernel ends (measured per launch on the 512-row projections: 0.1-1.0 us less, none slower).
 __device__ __forceinline__ void st4(float* p, f4 v, bool vec, int cnt) {
     if (vec) {
-        __builtin_nontemporal_store(v, reinterpret_cast<f4*>(p));
+        __builtin_nontemporal_store(v, reinterpret_cast<f4u*>(p));
         return;
     }
 #pragma unroll
@@ -228,7 +233,7 @@ __device__ __forceinline__ void st4(float* p, f4 v, bool vec, int cnt) {
 // Split-K partials, which the reduce launch reads next, are stored as ordinary lines.
 __device__ __forceinline__ void st4_keep(float* p, f4 v, bool vec, int cnt) {
     if (vec) {
-        *reinterpret_cast<f4*>(p) = v;
+        *reinterpret_cast<f4u*>(p) = v;
         return;
     }
 #pragma unroll
@@ -248,7 +253,9 @@ __device__ __forceinline__ f4 split_den(f4 r, const float* den, const float* bia
 }
 
 // ---- tile epilogue: ROWS x BN accumulator rows in LDS (Cs[ROWS][ldc]) -> outputs -----------------------
-template <int ROWS, int BN, int EPI, int T>
+// RAGGED: a 128-bit access wherever a row has four more columns, whatever N; without it, only where
+// N is a multiple of 4 (a uniform test: the per-lane one costs the 512-row launches about 1 us).
+template <int ROWS, int BN, int EPI, int T, bool RAGGED = false>
 __device__ void epilogue_rows(const float* Cs, int ldc, int64_t m0, int64_t n0, int64_t b, const Args& g) {
     constexpr int CPR = BN / 4;  // float4 columns per row
     const int tid = threadIdx.x;
@@ -273,7 +280,7 @@ __device__ void epilogue_rows(const float* Cs, int ldc, int64_t m0, int64_t n0, 
         const int64_t m = m0 + row, n = n0 + col;
         if (m >= g.M || n >= g.N) continue;
         const int cnt = g.N - n < 4 ? static_cast<int>(g.N - n) : 4;
-        const bool vec = g.vec_e && cnt == 4;
+        const bool vec = (RAGGED || g.vec_e) && cnt == 4;
         const f4 acc = *reinterpret_cast<const f4*>(Cs + row * ldc + col);
         if constexpr (EPI == PXK_EPI_STORE) {
             float* dst = C + m * g.c.ld + n;
@@ -622,7 +629,7 @@ __device__ __forceinline__ void tile_of(const Args& g, int& tm, int& tn, int& tz
 // With `rss` (PXK_PRO_RMS: `parts` partial sums of squares per tile row, `parts` x BM floats in LDS,
 // written before the call), every accumulator row is divided by its rms and the tile in the first
 // N column writes the rows' rms to g.row_rms.
-template <class C, int EPI>
+template <class C, int EPI, bool RAGGED = false>
 __device__ __forceinline__ void finish_tile(f4 (&acc)[C::TM][C::TN], float* smem, int ks, int wm, int wn, int lane,
                                             int tid, int64_t m0, int64_t n0, int64_t split, int64_t b, const Args& g,
                                             const float* rss = nullptr, int parts = 0) {
@@ -655,17 +662,16 @@ __device__ __forceinline__ void finish_tile(f4 (&acc)[C::TM][C::TN], float* smem
     }
     if (g.splits > 1) {  // raw partial tile -> workspace [split][batch][M][N]
         float* P = g.ws + ((split * g.batch + b) * g.M) * g.N;
-        const bool vec = (g.N % 4) == 0;
         for (int it = tid; it < BM * (BN / 4); it += C::NT) {
             const int row = it / (BN / 4), col = 4 * (it % (BN / 4));
             const int64_t m = m0 + row, n = n0 + col;
             if (m >= g.M || n >= g.N) continue;
             const int cnt = g.N - n < 4 ? static_cast<int>(g.N - n) : 4;
-            st4_keep(P + m * g.N + n, *reinterpret_cast<const f4*>(smem + row * LDC + col), vec && cnt == 4, cnt);
+            st4_keep(P + m * g.N + n, *reinterpret_cast<const f4*>(smem + row * LDC + col), g.vec_e && cnt == 4, cnt);
         }
         return;
     }
-    epilogue_rows<BM, BN, EPI, C::NT>(smem, LDC, m0, n0, b, g);
+    epilogue_rows<BM, BN, EPI, C::NT, RAGGED>(smem, LDC, m0, n0, b, g);
 }
 
 template <class C, bool TA, bool TB, int PRO, int EPI>
@@ -858,17 +864,20 @@ struct DirectChunk {
     f4 z[DS ? C::TM : 1];
     f4 zb;  // bias over k, the same for every A row
 
-    // An interior chunk (the whole 16-deep chunk of the tile lies inside both matrices) at K offset
-    // kc: unconditional loads.
+    // A chunk wholly inside K at K offset kc: unconditional loads. In an EDGE tile, rows and columns
+    // past the matrix read its last ones (never stored): 24 x 576 x 960 takes 9.4 us for 30 with each
+    // element guarded. Launches without edges run kernels without the clamp, whose arithmetic costs
+    // the 512-row products 1.3-1.6 us.
+    template <bool EDGE>
     __device__ __forceinline__ void load(const Args& g, const float* A, const float* Z, const float* ZB, const float* B,
                                          int64_t m0, int64_t n0, int64_t kc, int lane) {
         const int c = lane & 15, g4 = 4 * (lane >> 4);
 #pragma unroll
         for (int i = 0; i < C::TM; ++i) {
-            const int64_t m = m0 + 16 * i + c;
+            const int64_t m = EDGE ? min(m0 + 16 * i + c, g.M - 1) : m0 + 16 * i + c;
             if constexpr (!TA) {
-                a[i] = *reinterpret_cast<const f4*>(A + m * g.a.ld + kc + g4);
-                if constexpr (DS) z[i] = *reinterpret_cast<const f4*>(Z + m * g.z.ld + kc + g4);
+                a[i] = *reinterpret_cast<const f4u*>(A + m * g.a.ld + kc + g4);
+                if constexpr (DS) z[i] = *reinterpret_cast<const f4u*>(Z + m * g.z.ld + kc + g4);
             } else {
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
@@ -877,12 +886,12 @@ struct DirectChunk {
                 }
             }
         }
-        if constexpr (HB) zb = *reinterpret_cast<const f4*>(ZB + kc + g4);
+        if constexpr (HB) zb = *reinterpret_cast<const f4u*>(ZB + kc + g4);
 #pragma unroll
         for (int j = 0; j < C::TN; ++j) {
-            const int64_t n = n0 + 16 * j + c;
+            const int64_t n = EDGE ? min(n0 + 16 * j + c, g.N - 1) : n0 + 16 * j + c;
             if constexpr (TB) {
-                b[j] = *reinterpret_cast<const f4*>(B + n * g.b.ld + kc + g4);
+                b[j] = *reinterpret_cast<const f4u*>(B + n * g.b.ld + kc + g4);
             } else {
 #pragma unroll
                 for (int s = 0; s < 4; ++s) b[j][s] = B[(kc + g4 + s) * g.b.ld + n];
@@ -945,7 +954,9 @@ struct DirectChunk {
     }
 };
 
-template <class C, bool TA, bool TB, int PRO, int EPI>
+// EDGE: the launch has tiles that reach past M or N, or chunks past K. Without, none of their code is
+// in the kernel: these launches are short enough to feel their instruction fetches.
+template <class C, bool TA, bool TB, int PRO, int EPI, bool EDGE>
 __global__ void __launch_bounds__(C::NT) gemm_direct_kernel(const Args g) {
     static_assert(C::WM == 1 && C::WN == 1, "direct loads: every wave owns the whole tile");
     constexpr int BM = C::BM, BN = C::BN, TM = C::TM, TN = C::TN, KS = C::KS, PF = 3;
@@ -999,29 +1010,34 @@ __global__ void __launch_bounds__(C::NT) gemm_direct_kernel(const Args g) {
             if constexpr (kZB) ZB = obase(g.zb, b, g.inner, grp);
         }
     };
-    const bool interior = m0 + BM <= g.M && n0 + BN <= g.N && k_lo + 16 * static_cast<int64_t>(nch) <= g.K &&
-                          g.vec_a && g.vec_b;
-    if (nw > 0) {
-        if (interior) {
-            DirectChunk<C, TA, TB, PRO> ch[PF];
-            auto load = [&](auto S) {  // the cursor's chunk -> set S; the cursor stops at the last one
-                ch[S.value].load(g, A, Z, ZB, B, m0, n0, k_lo + 16 * kk, lane);
-                if (lu + 1 < nw) advance();
-            };
-            static_for<PF>([&](auto U) { load(U); });
-            for (int u0 = 0; u0 < nw; u0 += PF) {
-                static_for<PF>([&](auto U) {
-                    if (u0 + U.value < nw) ch[U.value].mma(acc, g.eps, ss);
-                    load(U);  // chunk u0 + U + PF (or the last one again)
-                });
-            }
-        } else {
-            DirectChunk<C, TA, TB, PRO> ch;
-            for (int u = 0; u < nw; ++u) {
-                ch.load_guarded(g, A, Z, ZB, B, m0, n0, k_lo + 16 * kk, lane);
-                ch.mma(acc, g.eps, ss);
-                if (u + 1 < nw) advance();
-            }
+    // Chunks past K (the last one of a ragged K) are loaded element by element: the wave's last chunk
+    // without k-groups; with them such chunks recur, and the wave loads every chunk that way.
+    int nf = nw;
+    if constexpr (EDGE) {
+        if (k_lo + 16 * static_cast<int64_t>(nch) > g.K && nw > 0)
+            nf = g.kgroups != 1 ? 0 : (first + KS * (nw - 1) == nch - 1 ? nw - 1 : nw);
+    }
+    if (nf > 0) {
+        DirectChunk<C, TA, TB, PRO> ch[PF];
+        auto load = [&](auto S) {  // the cursor's chunk -> set S; the cursor stops at the last one
+            ch[S.value].template load<EDGE>(g, A, Z, ZB, B, m0, n0, k_lo + 16 * kk, lane);
+            if (lu + 1 < nf) advance();
+        };
+        static_for<PF>([&](auto U) { load(U); });
+        for (int u0 = 0; u0 < nf; u0 += PF) {
+            static_for<PF>([&](auto U) {
+                if (u0 + U.value < nf) ch[U.value].mma(acc, g.eps, ss);
+                load(U);  // chunk u0 + U + PF (or the last one again)
+            });
+        }
+        if (EDGE && nf < nw) advance();
+    }
+    if constexpr (EDGE) {
+        DirectChunk<C, TA, TB, PRO> ch;
+        for (int u = nf; u < nw; ++u) {
+            ch.load_guarded(g, A, Z, ZB, B, m0, n0, k_lo + 16 * kk, lane);
+            ch.mma(acc, g.eps, ss);
+            if (u + 1 < nw) advance();
         }
     }
     if constexpr (PRO == PXK_PRO_RMS) {
@@ -1035,7 +1051,7 @@ __global__ void __launch_bounds__(C::NT) gemm_direct_kernel(const Args g) {
             if (lane < 16) s_rss[ks * BM + 16 * i + lane] = v;
         }
     }
-    finish_tile<C, EPI>(acc, smem, ks, 0, 0, lane, tid, m0, n0, split, b, g, PRO == PXK_PRO_RMS ? s_rss : nullptr, KS);
+    finish_tile<C, EPI, EDGE>(acc, smem, ks, 0, 0, lane, tid, m0, n0, split, b, g, PRO == PXK_PRO_RMS ? s_rss : nullptr, KS);
 }
 
 // The split partials of one 4-column group, added in split order. Eight loads are in flight at a
@@ -1073,7 +1089,7 @@ __global__ void __launch_bounds__(NT) splitk_reduce_kernel(const Args g) {
         // expressions, in the same order, as epilogue_rows.
         if (!mine || m >= g.M || n >= g.N) return;
         const int cnt = g.N - n < 4 ? static_cast<int>(g.N - n) : 4;
-        const bool vp = (g.N % 4) == 0 && cnt == 4, ve = g.vec_e && cnt == 4;
+        const bool vp = g.vec_e && cnt == 4, ve = vp;
         const int64_t inner = g.inner;
         const float* Y = g.y.p ? obase(g.y, b, inner, 0) + m * g.y.ld + n : nullptr;
         f4 x = ld4(obase(g.x, b, inner, 0) + m * g.x.ld + n, ve, cnt);
@@ -1104,7 +1120,7 @@ __global__ void __launch_bounds__(NT) splitk_reduce_kernel(const Args g) {
     f4 v = {0.f, 0.f, 0.f, 0.f};
     if (mine && m < g.M && n < g.N) {
         const int cnt = g.N - n < 4 ? static_cast<int>(g.N - n) : 4;
-        const bool vec = (g.N % 4) == 0 && cnt == 4;
+        const bool vec = g.vec_e && cnt == 4;
         const int64_t plane = g.batch * g.M * g.N;
         const float* P = g.ws + (b * g.M + m) * g.N + n;
         v = sum_partials(P, plane, g.splits, vec, cnt);
@@ -1298,17 +1314,436 @@ __global__ void __launch_bounds__(NT) skinny_nt_kernel(const Args g) {
     epilogue_rows<MB, kSkinnyBN, EPI, NT>(Cs, kSkinnyLDC, 0, n0, 0, g);
 }
 
+// ---- split-bf16 tiles -----------------------------------------------------------------------------
+// The fp32 product on the bf16 matrix units. Each operand element is split exactly into three bf16
+// parts, x = h + m + l (each the round-to-nearest of what is left: 8 + 8 + 8 significant bits and the
+// signs between them hold fp32's 24), and A B is summed as hh + (hm + mh + mm + hl + lh) with
+// v_mfma_f32_16x16x32_bf16: six products at 16 times the fp32 MFMA's rate, 2.67x its throughput. The
+// terms left out (ml, lm, ll) are below 2^-25 of a product; each part's product is exact in the fp32
+// accumulator, which rounds to nearest. hh has an accumulator of its own and the five small terms
+// another, so the large sum is rounded once per 32 K steps instead of once per 4: measured against
+// float64 over normal, positive and 4-sigma log-normal operands, the error is 0.3-1.0 of the fp32
+// MFMA's at K = 64 .. 8192 (relative 2-norm 4.3e-7 -> 1.4e-7 at K = 576, 1.6e-6 -> 5.7e-7 at 8192).
+// Infinities, NaN, overflow and results below 2^-90 (whose operands' low parts may lie under bf16's
+// subnormals) are not left to the split: a tile with any such element is computed again on the fp32
+// MFMA, so they come out as they always did.
+//
+// A stage of BK = 32 KS is loaded to registers as fp32 (one stage ahead), split once per element on its
+// way to LDS, and read back as ready MFMA fragments. LDS holds, per operand and part, 16-byte pieces of eight K values (4 q .. 4 q + 3 and 16 + 4 q .. of a 32-deep slice, so that the
+// loads of a row are contiguous across lanes; A and B agree on the order), placed free of bank
+// conflicts (SplitPanel::place).
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+
+constexpr float kSplitTiny = 8.077935669463161e-28f;  // 2^-90
+
+// Two floats to a packed bf16 pair (round to nearest even), and what is left of each.
+__device__ __forceinline__ uint32_t bf16_pair(float& a, float& b) {
+    const uint32_t p = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, bf2));
+    a -= __builtin_bit_cast(float, p << 16);
+    b -= __builtin_bit_cast(float, p & 0xffff0000u);
+    return p;
+}
+__device__ __forceinline__ void split8(float (&x)[8], u4 (&part)[3]) {
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part[p][j] = bf16_pair(x[2 * j], x[2 * j + 1]);
+}
+
+// NS register sets of prefetched stages. The large tile's stage is long enough for one, and two of its
+// workgroups share a CU on one LDS stage each; the small tiles' are not (a load takes about two of
+// their stages), and they double-buffer LDS for one barrier a stage.
+template <int BM_, int BN_, int WM_, int WN_, int KS_, int NS_>
+struct SCfg {
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, KS = KS_, NS = NS_;
+    static constexpr bool DB = NS > 1;
+    static constexpr int NT = 64 * WM * WN * KS;
+    static constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
+    static constexpr int BK = 32 * KS;
+    static constexpr int LDC = BN + 4;
+};
+
+using S128 = SCfg<128, 128, 2, 2, 1, 1>;
+using S64 = SCfg<64, 64, 2, 2, 1, 2>;
+
+// One operand panel of a stage: R rows of M (or N), BK deep, by T threads.
+template <int R, int BK, bool KC, int PRO, int T>
+struct SplitPanel {
+    static constexpr bool RMS = PRO == PXK_PRO_RMS;
+    static constexpr bool DS = PRO == PXK_PRO_DIV_STAB || PRO == kProStabBias;
+    static constexpr bool HB = PRO == kProStabBias;
+    static_assert(KC || !(DS || RMS), "prologue operands are K-contiguous");
+    static constexpr int KQ = BK / 8;
+    static constexpr int PLANE = R * KQ * 16;        // bytes of one part
+    static constexpr int SIZE = 3 * PLANE;
+    static constexpr int N = R * KQ, NV = (N + T - 1) / T;
+    static constexpr bool EVEN = N % T == 0;
+    float v[NV][8];
+    float z[DS ? NV : 1][8];
+    float zb[HB ? NV : 1][8];
+    float ss[RMS ? NV : 1] = {};
+
+    // Piece idx: its row of the panel and first K within the stage (the second four are 16 further).
+    __device__ __forceinline__ static void coords(int idx, int& r, int& k) {
+        const int q = KC ? idx % KQ : idx / R;
+        r = KC ? idx / KQ : idx % R;
+        k = 32 * (q / 4) + 4 * (q % 4);
+    }
+    // The thread's pieces' byte offsets from the stage's first element (KC: row r0, K k0; else row k0,
+    // column 0). Rows past the matrix read its last one: what they compute is never stored.
+    __device__ __forceinline__ static void lane_offsets(int64_t ld, int64_t mn, int64_t r0, unsigned (&off)[NV]) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            int r, k;
+            coords(static_cast<int>(threadIdx.x) + i * T, r, k);
+            const int64_t row = min(r0 + r, mn - 1);
+            off[i] = 4u * static_cast<unsigned>(KC ? (row - r0) * ld + k : k * ld + row);
+        }
+    }
+    __device__ __forceinline__ static void load8(const float* base, int64_t ld, unsigned off, float (&x)[8]) {
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, 0xFFFFFFFF, 0x00020000);
+        if constexpr (KC) {
+            const f4 a = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rs, static_cast<int>(off), 0, 0));
+            const f4 b = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rs, static_cast<int>(off), 64, 0));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                x[j] = a[j];
+                x[4 + j] = b[j];
+            }
+        } else {
+            const int step = 4 * static_cast<int>(ld);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                x[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, static_cast<int>(off), (j < 4 ? j : 12 + j) * step, 0));
+        }
+    }
+    // A stage wholly inside K.
+    __device__ __forceinline__ void issue(const float* A, int64_t lda, const unsigned (&off)[NV], const float* Z,
+                                          int64_t ldz, const unsigned (&offz)[DS ? NV : 1], const float* ZB) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            if (!EVEN && static_cast<int>(threadIdx.x) + i * T >= N) continue;
+            load8(A, lda, off[i], v[i]);
+            if constexpr (DS) load8(Z, ldz, offz[i], z[i]);
+            if constexpr (HB) {
+                int r, k;
+                coords(static_cast<int>(threadIdx.x) + i * T, r, k);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) zb[i][j] = ZB[k + (j < 4 ? j : 12 + j)];
+            }
+        }
+    }
+    // Any stage, element by element; zeros past K. A, Z and ZB at the operand's first element.
+    __device__ __forceinline__ void issue_any(const float* A, int64_t lda, const float* Z, int64_t ldz, const float* ZB,
+                                              int64_t mn, int64_t r0, int64_t k0, int64_t K) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            int r, k;
+            coords(static_cast<int>(threadIdx.x) + i * T, r, k);
+            const int64_t row = min(r0 + r, mn - 1);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int64_t kk = k0 + k + (j < 4 ? j : 12 + j);
+                const bool in = kk < K;
+                v[i][j] = in ? (KC ? A[row * lda + kk] : A[kk * lda + row]) : 0.0f;
+                if constexpr (DS) z[i][j] = in ? Z[row * ldz + kk] : 1.0f;
+                if constexpr (HB) zb[i][j] = in ? ZB[kk] : 0.0f;
+            }
+        }
+    }
+    __device__ __forceinline__ void commit(char* lds, float eps) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int idx = static_cast<int>(threadIdx.x) + i * T;
+            if (!EVEN && idx >= N) continue;
+            if constexpr (RMS) {
+#pragma unroll
+                for (int j = 0; j < 8; j += 4)
+                    ss[i] += v[i][j] * v[i][j] + v[i][j + 1] * v[i][j + 1] + v[i][j + 2] * v[i][j + 2] + v[i][j + 3] * v[i][j + 3];
+            }
+            if constexpr (DS) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    v[i][j] = v[i][j] * __builtin_amdgcn_rcpf(stab(HB ? z[i][j] + zb[i][j] : z[i][j], eps));
+            }
+            u4 part[3];
+            split8(v[i], part);
+            char* p = lds + (KC ? place(idx / KQ, idx % KQ) : place(idx % R, idx / R));
+#pragma unroll
+            for (int s = 0; s < 3; ++s) *reinterpret_cast<u4*>(p + s * PLANE) = part[s];
+        }
+    }
+    // Byte offset of row r's piece q: 16 x 32 blocks in fragment order (four runs of 16 rows' pieces, so
+    // a fragment is 1024 contiguous bytes), each run's rows permuted by its piece and slice so that the
+    // pieces of a row, which adjacent lanes write, lie in different banks. A 128-bit read takes rows
+    // 0-3 and 12-15 of one run together with rows 4-11 of the next: runs 0 and 1, and 2 and 3, are
+    // permuted alike in that respect.
+    __device__ __forceinline__ static int place(int r, int q) {
+        return ((((r >> 4) * KQ + q) << 4) + ((r & 15) ^ ((-q & 3) << 2) ^ ((q >> 2) & 3))) << 4;
+    }
+    // Part s of the 16-row fragment at row `off` for K slice ks.
+    __device__ __forceinline__ static bf8 fragment(const char* lds, int s, int ks, int off, int lane) {
+        return __builtin_bit_cast(bf8, *reinterpret_cast<const u4*>(lds + s * PLANE + place(off + (lane & 15), 4 * ks + (lane >> 4))));
+    }
+};
+
+// The tile on the fp32 MFMA, straight from memory: for the tiles the split does not settle.
+template <class C, bool TA, bool TB, int PRO>
+__device__ __forceinline__ void fp32_tile(const Args& g, f4 (&acc)[C::TM][C::TN], int64_t m0, int64_t n0, int64_t b,
+                                          int64_t k_lo, int nkb, int t0, int t1, int ks, int lane) {
+    constexpr bool DS = PRO == PXK_PRO_DIV_STAB || PRO == kProStabBias;
+    const int c = lane & 15, kl = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+        for (int j = 0; j < C::TN; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int t = t0; t < t1; ++t) {
+        const int grp = t / nkb;
+        const float* A = obase(g.a, b, g.inner, grp);
+        const float* B = obase(g.b, b, g.inner, grp);
+        const float* Z = DS ? obase(g.z, b, g.inner, grp) : nullptr;
+        const float* ZB = PRO == kProStabBias ? obase(g.zb, b, g.inner, grp) : nullptr;
+        const int64_t k0 = k_lo + static_cast<int64_t>(t - grp * nkb) * C::BK + 32 * ks;
+#pragma unroll 1
+        for (int kk = kl; kk < 32; kk += 4) {
+            const int64_t k = k0 + kk;
+            float a[C::TM], bb[C::TN];
+#pragma unroll
+            for (int i = 0; i < C::TM; ++i) {
+                const int64_t m = min(m0 + 16 * i + c, g.M - 1);
+                a[i] = k < g.K ? (TA ? A[k * g.a.ld + m] : A[m * g.a.ld + k]) : 0.0f;
+                if constexpr (DS) {
+                    const float z = k < g.K ? (TA ? Z[k * g.z.ld + m] : Z[m * g.z.ld + k]) : 1.0f;
+                    a[i] *= __builtin_amdgcn_rcpf(stab(ZB && k < g.K ? z + ZB[k] : z, g.eps));
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < C::TN; ++j) {
+                const int64_t n = min(n0 + 16 * j + c, g.N - 1);
+                bb[j] = k < g.K ? (TB ? B[n * g.b.ld + k] : B[k * g.b.ld + n]) : 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], bb[j], acc[i][j], 0, 0, 0);
+        }
+    }
+}
+
+template <class C, bool TA, bool TB, int PRO, int EPI>
+__global__ void __launch_bounds__(C::NT, 2) gemm_split_kernel(const Args g) {
+    constexpr int BM = C::BM, BN = C::BN, BK = C::BK, TM = C::TM, TN = C::TN;
+    using PA = SplitPanel<BM, BK, !TA, PRO, C::NT>;
+    using PB = SplitPanel<BN, BK, TB, PXK_PRO_NONE, C::NT>;
+    constexpr int STAGE = PA::SIZE + PB::SIZE, BUFS = C::DB ? 2 : 1;
+    constexpr int PART = 4 * C::KS * BM * C::LDC, LDS = BUFS * STAGE > PART ? BUFS * STAGE : PART;
+    __shared__ __attribute__((aligned(16))) char smem[LDS];
+    __shared__ float s_rss[PRO == PXK_PRO_RMS ? BM : 1];
+    constexpr bool kZ = PRO == PXK_PRO_DIV_STAB || PRO == kProStabBias, kZB = PRO == kProStabBias;
+
+    int tm, tn, tz;
+    tile_of(g, tm, tn, tz);
+    const int64_t m0 = static_cast<int64_t>(tm) * BM, n0 = static_cast<int64_t>(tn) * BN;
+    const int64_t split = tz % g.splits, b = tz / g.splits;
+    if (g.causal == PXK_CAUSAL_TRI && n0 > m0 + BM - 1) return;  // tile strictly above the diagonal
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ks = wave / (C::WM * C::WN), wmn = wave % (C::WM * C::WN);
+    const int wm = (wmn / C::WN) * (BM / C::WM), wn = (wmn % C::WN) * (BN / C::WN);
+
+    const int64_t k_lo = k_first(g, m0), k_hi = k_end(g, m0, BM);
+    const int nkb = k_hi > k_lo ? static_cast<int>((k_hi - k_lo + BK - 1) / BK) : 0;
+    const int total = nkb * static_cast<int>(g.kgroups);
+    const int per = (total + g.splits - 1) / g.splits;
+    const int t0 = min(static_cast<int>(split) * per, total), t1 = min(t0 + per, total);
+
+    f4 acc[TM][TN], low[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = low[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+
+    constexpr int NS = C::NS;
+    PA pa[NS];
+    PB pb[NS];
+    unsigned offa[PA::NV], offb[PB::NV], offz[kZ ? PA::NV : 1];
+    PA::lane_offsets(g.a.ld, g.M, m0, offa);
+    PB::lane_offsets(g.b.ld, g.N, n0, offb);
+    if constexpr (kZ) PA::lane_offsets(g.z.ld, g.M, m0, offz);
+
+    int grp = nkb > 0 ? t0 / nkb : 0, kb = nkb > 0 ? t0 % nkb : 0;
+    const float* A = obase(g.a, b, g.inner, grp);
+    const float* B = obase(g.b, b, g.inner, grp);
+    const float* Z = kZ ? obase(g.z, b, g.inner, grp) : nullptr;
+    const float* ZB = kZB ? obase(g.zb, b, g.inner, grp) : nullptr;
+    auto advance = [&]() {
+        if (++kb == nkb) {  // next k-group: rebase the operands
+            kb = 0;
+            ++grp;
+            A = obase(g.a, b, g.inner, grp);
+            B = obase(g.b, b, g.inner, grp);
+            if constexpr (kZ) Z = obase(g.z, b, g.inner, grp);
+            if constexpr (kZB) ZB = obase(g.zb, b, g.inner, grp);
+        }
+    };
+    const int whole = static_cast<int>((g.K - k_lo) / BK);  // stages inside K, from k_lo
+    int nf = (g.kgroups == 1 ? min(t1, whole) : (nkb <= whole ? t1 : t0)) - t0;
+    // The lanes' 32-bit offsets have to reach the panel's last row.
+    const int64_t ldmax = max(max(g.a.ld, g.b.ld), kZ ? g.z.ld : int64_t{0});
+    if (ldmax >= (int64_t{1} << 22)) nf = 0;
+    int lt = 0;  // stages issued
+    auto issue = [&](auto S) {  // the cursor's stage, wholly inside K, into set S; the cursor stops at the last one
+        const int64_t k0 = k_lo + static_cast<int64_t>(kb) * BK;
+        pa[S.value].issue(!TA ? A + m0 * g.a.ld + k0 : A + k0 * g.a.ld, g.a.ld, offa,
+                          kZ ? Z + m0 * g.z.ld + k0 : nullptr, g.z.ld, offz, kZB ? ZB + k0 : nullptr);
+        const unsigned none[1] = {0};
+        pb[S.value].issue(TB ? B + n0 * g.b.ld + k0 : B + k0 * g.b.ld, g.b.ld, offb, nullptr, 0, none, nullptr);
+        if (++lt < nf) advance();
+    };
+    auto commit = [&](auto S, int buf) {
+        pa[S.value].commit(smem + buf * STAGE, g.eps);
+        pb[S.value].commit(smem + buf * STAGE + PA::SIZE, g.eps);
+    };
+    auto compute = [&](int buf) {
+        const char* As = smem + buf * STAGE;
+        const char* Bs = As + PA::SIZE;
+        bf8 a[3][TM];
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+#pragma unroll
+            for (int i = 0; i < TM; ++i) a[s][i] = PA::fragment(As, s, ks, wm + 16 * i, lane);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            bf8 bb[3];
+#pragma unroll
+            for (int s = 0; s < 3; ++s) bb[s] = PB::fragment(Bs, s, ks, wn + 16 * j, lane);
+            constexpr int pairs[5][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}};
+#pragma unroll
+            for (int p = 0; p < 5; ++p)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+                    low[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[pairs[p][0]][i], bb[pairs[p][1]], low[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0][i], bb[0], acc[i][j], 0, 0, 0);
+        }
+    };
+
+    // Full stages, the next NS in flight over the current one's MFMAs. Loads are unconditional (past the
+    // last stage it is loaded again, into a set nobody commits).
+    using I0 = std::integral_constant<int, 0>;
+    if (nf > NS && C::DB) {
+        issue(I0{});
+        commit(I0{}, 0);
+        static_for<NS>([&](auto U) { issue(std::integral_constant<int, (U.value + 1) % NS>{}); });
+        __syncthreads();
+        const int main_iters = (nf - 2) / NS * NS;  // a multiple of NS, >= nf - NS - 1
+        for (int tb = 0; tb < main_iters; tb += NS) {
+            static_for<NS>([&](auto U) {
+                using Next = std::integral_constant<int, (U.value + 1) % NS>;
+                const int t = tb + U.value;
+                commit(Next{}, (t + 1) & 1);  // that buffer was last read by stage t - 1, before the barrier
+                issue(Next{});
+                compute(t & 1);
+                __syncthreads();
+            });
+        }
+        static_for<NS + 1>([&](auto U) {  // the last 2 .. NS + 1 stages: already in flight
+            using Next = std::integral_constant<int, (U.value + 1) % NS>;
+            const int t = main_iters + U.value;
+            if (t < nf) {
+                if (t + 1 < nf) commit(Next{}, (t + 1) & 1);
+                compute(t & 1);
+                __syncthreads();
+            }
+        });
+    } else if (C::DB && nf > 0) {  // no more stages than sets: all in flight at once
+        static_for<NS>([&](auto U) {
+            if (U.value < nf) issue(U);
+        });
+        static_for<NS>([&](auto U) {
+            if (U.value < nf) {
+                commit(U, U.value & 1);
+                __syncthreads();
+                compute(U.value & 1);
+            }
+        });
+        __syncthreads();
+    } else if (nf > 0) {
+        issue(I0{});
+        for (int t = 0; t < nf; ++t) {
+            commit(I0{}, 0);
+            __syncthreads();
+            issue(I0{});
+            compute(0);
+            __syncthreads();
+        }
+    }
+    // The ragged last stage (with k-groups it would recur, so those run stage by stage unless K is a
+    // multiple of BK).
+    if (nf > 0 && nf < t1 - t0) advance();
+    for (int t = max(nf, 0); t < t1 - t0; ++t) {
+        const int64_t k0 = k_lo + static_cast<int64_t>(kb) * BK;
+        pa[0].issue_any(A, g.a.ld, Z, g.z.ld, ZB, g.M, m0, k0, g.K);
+        pb[0].issue_any(B, g.b.ld, nullptr, 0, nullptr, g.N, n0, k0, g.K);
+        advance();
+        commit(I0{}, 0);
+        __syncthreads();
+        compute(0);
+        __syncthreads();
+    }
+
+    bool redo = false;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            acc[i][j] += low[i][j];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float v = fabsf(acc[i][j][r]);
+                redo |= !(v <= 3.4028234663852886e38f) || (v < kSplitTiny && v != 0.0f);
+            }
+        }
+    if (__syncthreads_or(redo))
+        fp32_tile<C, TA, TB, PRO>(g, acc, m0 + wm, n0 + wn, b, k_lo, nkb, t0, t1, ks, lane);
+
+    if constexpr (PRO == PXK_PRO_RMS) {
+        // Each A element was committed once; the KQ consecutive threads of a row add their sums.
+#pragma unroll
+        for (int i = 0; i < PA::NV; ++i) {
+            float v = 0.0f;
+            static_for<NS>([&](auto S) { v += pa[S.value].ss[i]; });
+#pragma unroll
+            for (int o = 1; o < PA::KQ; o <<= 1) v += __shfl_xor(v, o, 64);
+            const int idx = tid + i * C::NT;
+            if (idx < PA::N && idx % PA::KQ == 0) s_rss[idx / PA::KQ] = v;
+        }
+    }
+    finish_tile<C, EPI, true>(acc, reinterpret_cast<float*>(smem), ks, wm, wn, lane, tid, m0, n0, split, b, g,
+                        PRO == PXK_PRO_RMS ? s_rss : nullptr, 1);
+}
+
 #define PXK_KSET(TA, TB, P, EPI)                                                                    \
     {gemm_kernel<C128, TA, TB, P, EPI>, gemm_kernel<C64, TA, TB, P, EPI>, gemm_kernel<C32x64, TA, TB, P, EPI>, \
-     gemm_kernel<C32, TA, TB, P, EPI>, gemm_direct_kernel<C32x64, TA, TB, P, EPI>,                         \
-     gemm_direct_kernel<C32, TA, TB, P, EPI>, gemm_direct_kernel<C32x48, TA, TB, P, EPI>,                  \
-     gemm_kernel<C32x48, TA, TB, P, EPI>}
+     gemm_kernel<C32, TA, TB, P, EPI>, gemm_direct_kernel<C32x64, TA, TB, P, EPI, false>,                  \
+     gemm_direct_kernel<C32, TA, TB, P, EPI, false>, gemm_direct_kernel<C32x48, TA, TB, P, EPI, false>,    \
+     gemm_kernel<C32x48, TA, TB, P, EPI>, gemm_split_kernel<S128, TA, TB, P, EPI>,                         \
+     gemm_split_kernel<S64, TA, TB, P, EPI>}
+#define PXK_EDGES(TA, TB, P, EPI)                                                                         \
+    {gemm_direct_kernel<C32x64, TA, TB, P, EPI, true>, gemm_direct_kernel<C32, TA, TB, P, EPI, true>,     \
+     gemm_direct_kernel<C32x48, TA, TB, P, EPI, true>}
 #define PXK_GEMM_ENTRY(TA, TB, PRO, EPI)                                                                   \
     Entry {                                                                                                \
         TA, TB, PRO, EPI, {PXK_KSET(TA, TB, PRO, EPI), PXK_KSET(TA, TB, (PRO == PXK_PRO_DIV_STAB ? kProStabBias : PRO), EPI)}, \
             {splitk_reduce_kernel<128, EPI>, splitk_reduce_kernel<64, EPI>, splitk_reduce_kernel<64, EPI>, \
              splitk_reduce_kernel<32, EPI>, splitk_reduce_kernel<64, EPI>, splitk_reduce_kernel<32, EPI>,   \
-             splitk_reduce_kernel<48, EPI>, splitk_reduce_kernel<48, EPI>},                                 \
+             splitk_reduce_kernel<48, EPI>, splitk_reduce_kernel<48, EPI>,                                  \
+             splitk_reduce_kernel<128, EPI>, splitk_reduce_kernel<64, EPI>},                                \
+            {PXK_EDGES(TA, TB, PRO, EPI), PXK_EDGES(TA, TB, (PRO == PXK_PRO_DIV_STAB ? kProStabBias : PRO), EPI)}, \
     }
 
 constexpr int skinny_rows(int mb) { return mb == 4 ? 16 : (mb == 8 ? 16 : 8); }

@@ -37,7 +37,7 @@ class GemmDesc(ctypes.Structure):
                 ("tile", ctypes.c_int32), ("workspace", c_vp), ("workspace_bytes", ctypes.c_size_t),
                 ("rope_cols", c_i64), ("gate_act", ctypes.c_int32), ("reserved", ctypes.c_int32),
                 ("c2_den", Operand), ("c2_den_bias", Operand), ("x_rms", c_vp), ("x_gamma", c_vp), ("row_rms", c_vp),
-                ("norm_eps", ctypes.c_float), ("reserved2", ctypes.c_int32)]
+                ("norm_eps", ctypes.c_float), ("denominator", ctypes.c_int32)]
 
 
 CAUSAL_NONE, CAUSAL_TRI, CAUSAL_K_LE_M, CAUSAL_K_GE_M = 0, 1, 2, 3
@@ -47,6 +47,7 @@ PRO_NONE, PRO_DIV_STAB, PRO_RMS = 0, 1, 2
 TILE_AUTO, TILE_128x128, TILE_64x64, TILE_32x64, TILE_32x32, TILE_32x64_DIRECT, TILE_32x32_DIRECT, TILE_SKINNY = range(8)
 TILE_32x48_DIRECT = 8
 TILE_32x48 = 9
+TILE_128x128_SPLIT, TILE_64x64_SPLIT = 10, 11
 
 # (name, restype, argtypes) of every pxk entry point; `p` = device pointer (void*), `i` = int64,
 # `f` = float, `n` = int, `s` = size_t.
