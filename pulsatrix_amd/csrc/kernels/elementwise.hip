@@ -313,13 +313,48 @@ __global__ void __launch_bounds__(kThreads) accumulate_rows_kernel(const float* 
     out[j] = acc;
 }
 
-__global__ void __launch_bounds__(kThreads) column_sums_kernel(const float* in, float* out, int64_t rows, int64_t cols,
-                                                               float beta) {
+// Few rows: one thread per column, in row order.
+__global__ void __launch_bounds__(kThreads) column_sums_short_kernel(const float* in, float* out, int64_t rows,
+                                                                     int64_t cols, float beta) {
     const int64_t j = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (j >= cols) return;
     float acc = 0.0f;
     for (int64_t r = 0; r < rows; ++r) acc += in[r * cols + j];
     out[j] = (beta == 0.0f) ? acc : beta * out[j] + acc;
+}
+
+// Bound by reading `in` once. A workgroup owns 16 columns (64-byte row segments, so that 2048 columns
+// still give 128 workgroups) and walks the rows 64 at a time with eight loads in flight per thread;
+// the 64 row lanes' sums meet in a fixed order: the four of a wave by shuffles, then the 16 waves
+// through LDS. 4096 x 2048: 942 us with one thread per column, 13 us so (2.6 TB/s).
+constexpr int kSumCols = 16, kSumThreads = 1024, kSumRows = kSumThreads / kSumCols;
+__global__ void __launch_bounds__(kSumThreads) column_sums_kernel(const float* in, float* out, int64_t rows, int64_t cols,
+                                                                  float beta) {
+    __shared__ float part[kSumThreads / kWave][kSumCols];
+    const int c = threadIdx.x % kSumCols, lane = threadIdx.x & (kWave - 1);
+    const int64_t j = static_cast<int64_t>(blockIdx.x) * kSumCols + c;
+    const float* p = in + (j < cols ? j : cols - 1);
+    float acc = 0.0f;
+    int64_t r = threadIdx.x / kSumCols;
+    constexpr int U = 8;
+    for (; r + (U - 1) * kSumRows < rows; r += U * kSumRows) {
+        float v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = p[(r + u * kSumRows) * cols];
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc += v[u];
+    }
+    for (; r < rows; r += kSumRows) acc += p[r * cols];
+    acc += __shfl_xor(acc, 16, kWave);
+    acc += __shfl_xor(acc, 32, kWave);
+    if (lane < kSumCols) part[threadIdx.x / kWave][c] = acc;
+    __syncthreads();
+    if (threadIdx.x < kSumCols && j < cols) {
+        float t = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kSumThreads / kWave; ++w) t += part[w][c];
+        out[j] = (beta == 0.0f) ? t : beta * out[j] + t;
+    }
 }
 
 __global__ void __launch_bounds__(kThreads) gather_kernel(const float* table, const float* idx, float* out,
@@ -493,8 +528,13 @@ int pxk_accumulate_rows(const float* in, float* out, int64_t rows, int64_t cols,
 int pxk_column_sums(const float* in, float* out, int64_t rows, int64_t cols, float beta, void* stream) {
     if (rows < 0 || cols < 0) return fail(PXK_ERR_INVALID, "pxk_column_sums: negative size");
     if (cols == 0) return PXK_OK;
-    PXK_LAUNCH(column_sums_kernel, dim3(static_cast<unsigned>(cdiv(cols, kThreads))), dim3(kThreads), 0,
-                       S(stream), in, out, rows, cols, beta);
+    // Up to a quarter of a step of rows, most row lanes would be idle.
+    if (rows <= kSumRows / 4)
+        PXK_LAUNCH(column_sums_short_kernel, dim3(static_cast<unsigned>(cdiv(cols, kThreads))), dim3(kThreads), 0,
+                   S(stream), in, out, rows, cols, beta);
+    else
+        PXK_LAUNCH(column_sums_kernel, dim3(static_cast<unsigned>(cdiv(cols, kSumCols))), dim3(kSumThreads), 0,
+                   S(stream), in, out, rows, cols, beta);
     return launched("pxk_column_sums");
 }
 
