@@ -8,6 +8,7 @@
 #include <cstring>
 
 #include "common.hpp"
+#include "held_rows.hpp"
 
 namespace pxk {
 namespace {
@@ -196,6 +197,35 @@ __global__ void __launch_bounds__(kThreads) softmax_kernel(const float* in, floa
     for (int64_t j = lane; j < cols; j += kWave) s += expf(x[j] - mx);
     s = wave_sum(s);
     for (int64_t j = lane; j < cols; j += kWave) y[j] = expf(x[j] - mx) / s;
+}
+
+// The same from registers (held_rows.hpp), one exponential an element.
+template <class Shape>
+__global__ void __launch_bounds__(kHeldThreads) softmax_held_kernel(const float* in, float* out, int64_t rows,
+                                                                    int64_t cols) {
+    const HeldRow<Shape> h(cols);
+    if (h.row >= rows) return;
+    typename HeldRow<Shape>::vec v[Shape::NV];
+    h.load(in + h.row * cols, v);
+    float mx = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < Shape::NV; ++j)
+#pragma unroll
+        for (int i = 0; i < Shape::V; ++i) mx = fmaxf(mx, v[j][i]);
+    mx = held_max<Shape::T>(mx);
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < Shape::NV; ++j)
+#pragma unroll
+        for (int i = 0; i < Shape::V; ++i) {
+            v[j][i] = expf(v[j][i] - mx);
+            s += h.live(j) ? v[j][i] : 0.0f;
+        }
+    s = held_sum<Shape::T>(s);
+    float* y = out + h.row * cols;
+#pragma unroll
+    for (int j = 0; j < Shape::NV; ++j)
+        if (h.live(j)) h.store(y, j, v[j] / s);
 }
 
 // ---- lrp_softmax_rows (lrp_math.hpp:89-98) ----------------------------------------------------
@@ -667,7 +697,12 @@ int pxk_rms_norm_add(const float* x, const float* a, const float* gamma_a, float
 int pxk_softmax_rows(const float* in, float* out, int64_t rows, int64_t cols, void* stream) {
     int rc;
     if (!sizes_ok("pxk_softmax_rows", rows, cols, &rc)) return rc;
-    PXK_LAUNCH(softmax_kernel, dim3(rows_grid(rows)), dim3(kThreads), 0, S(stream), in, out, rows, cols);
+    const bool held = with_held_shape(cols, aligned16(in) && aligned16(out), [&](auto shape) {
+        using Shape = decltype(shape);
+        PXK_LAUNCH((softmax_held_kernel<Shape>), held_grid<Shape>(rows), dim3(kHeldThreads), 0, S(stream), in, out, rows,
+                   cols);
+    });
+    if (!held) PXK_LAUNCH(softmax_kernel, dim3(rows_grid(rows)), dim3(kThreads), 0, S(stream), in, out, rows, cols);
     return launched("pxk_softmax_rows");
 }
 

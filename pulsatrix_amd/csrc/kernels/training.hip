@@ -10,6 +10,7 @@
 #include <cstdint>
 
 #include "common.hpp"
+#include "held_rows.hpp"
 
 namespace pxk {
 namespace {
@@ -84,6 +85,26 @@ __global__ void __launch_bounds__(kThreads) softmax_backward_kernel(const float*
     for (int64_t j = lane; j < cols; j += kWave) dx[row * cols + j] = yr[j] * (gr[j] - dot);
 }
 
+// The same from registers (held_rows.hpp).
+template <class Shape>
+__global__ void __launch_bounds__(kHeldThreads) softmax_backward_held_kernel(const float* y, const float* dy, float* dx,
+                                                                             int64_t rows, int64_t cols) {
+    const HeldRow<Shape> h(cols);
+    if (h.row >= rows) return;
+    typename HeldRow<Shape>::vec yv[Shape::NV], gv[Shape::NV];
+    h.load(y + h.row * cols, yv);
+    h.load(dy + h.row * cols, gv);
+    float dot = 0.0f;
+#pragma unroll
+    for (int j = 0; j < Shape::NV; ++j)
+#pragma unroll
+        for (int i = 0; i < Shape::V; ++i) dot += h.live(j) ? yv[j][i] * gv[j][i] : 0.0f;
+    dot = held_sum<Shape::T>(dot);
+#pragma unroll
+    for (int j = 0; j < Shape::NV; ++j)
+        if (h.live(j)) h.store(dx + h.row * cols, j, yv[j] * (gv[j] - dot));
+}
+
 // rms_norm_backward (row_math.hpp:75-86): gamma_terms = g x / rms; grad_in = g gamma / rms
 // - x / (D rms^3) sum(g gamma x).
 __global__ void __launch_bounds__(kThreads) rms_backward_kernel(const float* gy, const float* gamma, const float* x,
@@ -99,6 +120,34 @@ __global__ void __launch_bounds__(kThreads) rms_backward_kernel(const float* gy,
         gterms[off + j] = gy[off + j] * x[off + j] / rms;
         gx[off + j] = gy[off + j] * gamma[j] / rms - (x[off + j] / (D * rms * rms * rms)) * dot;
     }
+}
+
+// The same from registers (held_rows.hpp).
+template <class Shape>
+__global__ void __launch_bounds__(kHeldThreads) rms_backward_held_kernel(const float* gy, const float* gamma,
+                                                                         const float* x, const float* row_rms, float* gx,
+                                                                         float* gterms, int64_t rows, int64_t cols) {
+    const HeldRow<Shape> h(cols);
+    if (h.row >= rows) return;
+    typename HeldRow<Shape>::vec gv[Shape::NV], xv[Shape::NV], wv[Shape::NV];
+    const int64_t off = h.row * cols;
+    h.load(gy + off, gv);
+    h.load(x + off, xv);
+    h.load(gamma, wv);
+    const float rms = row_rms[h.row], D = static_cast<float>(cols);
+    float dot = 0.0f;
+#pragma unroll
+    for (int j = 0; j < Shape::NV; ++j)
+#pragma unroll
+        for (int i = 0; i < Shape::V; ++i) dot += h.live(j) ? gv[j][i] * wv[j][i] * xv[j][i] : 0.0f;
+    dot = held_sum<Shape::T>(dot);
+    const float den = D * rms * rms * rms;
+#pragma unroll
+    for (int j = 0; j < Shape::NV; ++j)
+        if (h.live(j)) {
+            h.store(gterms + off, j, gv[j] * xv[j] / rms);
+            h.store(gx + off, j, gv[j] * wv[j] / rms - (xv[j] / den) * dot);
+        }
 }
 
 // layer_norm_forward (row_math.hpp:15-38): mean, then the mean of squared deviations, std =
@@ -160,6 +209,29 @@ __global__ void __launch_bounds__(kThreads) logsumexp_kernel(const float* in, fl
     for (int64_t j = lane; j < cols; j += kWave) s += expf(x[j] - m);
     s = wave_sum(s);
     if (lane == 0) out[row] = m + logf(s);
+}
+
+// The same from registers (held_rows.hpp).
+template <class Shape>
+__global__ void __launch_bounds__(kHeldThreads) logsumexp_held_kernel(const float* in, float* out, int64_t rows,
+                                                                      int64_t cols) {
+    const HeldRow<Shape> h(cols);
+    if (h.row >= rows) return;
+    typename HeldRow<Shape>::vec v[Shape::NV];
+    h.load(in + h.row * cols, v);
+    float m = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < Shape::NV; ++j)
+#pragma unroll
+        for (int i = 0; i < Shape::V; ++i) m = fmaxf(m, v[j][i]);
+    m = held_max<Shape::T>(m);
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < Shape::NV; ++j)
+#pragma unroll
+        for (int i = 0; i < Shape::V; ++i) s += h.live(j) ? expf(v[j][i] - m) : 0.0f;
+    s = held_sum<Shape::T>(s);
+    if (h.t == 0) out[h.row] = m + logf(s);
 }
 
 // scatter_add_rows (cpu_backend.cpp:468-475): table[idx[i]] += src[i] for i ascending. A thread
@@ -333,7 +405,13 @@ int pxk_elementwise_backward(int op, const float* x, const float* grad_out, floa
 int pxk_softmax_rows_backward(const float* y, const float* dy, float* dx, int64_t rows, int64_t cols, void* stream) {
     int rc;
     if (bad_rows("pxk_softmax_rows_backward", rows, cols, &rc)) return rc;
-    PXK_LAUNCH(softmax_backward_kernel, dim3(rows_grid(rows)), dim3(kThreads), 0, S(stream), y, dy, dx, rows, cols);
+    const bool held = with_held_shape(cols, aligned16(y) && aligned16(dy) && aligned16(dx), [&](auto shape) {
+        using Shape = decltype(shape);
+        PXK_LAUNCH((softmax_backward_held_kernel<Shape>), held_grid<Shape>(rows), dim3(kHeldThreads), 0, S(stream), y, dy,
+                   dx, rows, cols);
+    });
+    if (!held)
+        PXK_LAUNCH(softmax_backward_kernel, dim3(rows_grid(rows)), dim3(kThreads), 0, S(stream), y, dy, dx, rows, cols);
     return launched("pxk_softmax_rows_backward");
 }
 
@@ -341,8 +419,15 @@ int pxk_rms_norm_backward(const float* grad_out, const float* gamma, const float
                           float* grad_in, float* gamma_terms, int64_t rows, int64_t cols, void* stream) {
     int rc;
     if (bad_rows("pxk_rms_norm_backward", rows, cols, &rc)) return rc;
-    PXK_LAUNCH(rms_backward_kernel, dim3(rows_grid(rows)), dim3(kThreads), 0, S(stream), grad_out, gamma, in, row_rms,
-               grad_in, gamma_terms, rows, cols);
+    const bool vec = aligned16(grad_out) && aligned16(gamma) && aligned16(in) && aligned16(grad_in) && aligned16(gamma_terms);
+    const bool held = with_held_shape(cols, vec, [&](auto shape) {
+        using Shape = decltype(shape);
+        PXK_LAUNCH((rms_backward_held_kernel<Shape>), held_grid<Shape>(rows), dim3(kHeldThreads), 0, S(stream), grad_out,
+                   gamma, in, row_rms, grad_in, gamma_terms, rows, cols);
+    });
+    if (!held)
+        PXK_LAUNCH(rms_backward_kernel, dim3(rows_grid(rows)), dim3(kThreads), 0, S(stream), grad_out, gamma, in, row_rms,
+                   grad_in, gamma_terms, rows, cols);
     return launched("pxk_rms_norm_backward");
 }
 
@@ -368,7 +453,12 @@ int pxk_logsumexp_rows(const float* in, float* out, int64_t rows, int64_t cols, 
     int rc;
     if (cols == 0 && rows > 0) return fail(PXK_ERR_INVALID, "pxk_logsumexp_rows: empty rows");
     if (bad_rows("pxk_logsumexp_rows", rows, cols, &rc)) return rc;
-    PXK_LAUNCH(logsumexp_kernel, dim3(rows_grid(rows)), dim3(kThreads), 0, S(stream), in, out, rows, cols);
+    const bool held = with_held_shape(cols, aligned16(in), [&](auto shape) {
+        using Shape = decltype(shape);
+        PXK_LAUNCH((logsumexp_held_kernel<Shape>), held_grid<Shape>(rows), dim3(kHeldThreads), 0, S(stream), in, out,
+                   rows, cols);
+    });
+    if (!held) PXK_LAUNCH(logsumexp_kernel, dim3(rows_grid(rows)), dim3(kThreads), 0, S(stream), in, out, rows, cols);
     return launched("pxk_logsumexp_rows");
 }
 
