@@ -45,12 +45,18 @@ def test_held_rows(cols, offset):
     _call("pxk_logsumexp_rows", G.ptr(dx), G.ptr(lse), rows, cols)
     _call("pxk_softmax_rows_backward", G.ptr(dx), G.ptr(dg), G.ptr(dp), rows, cols)
     _call("pxk_rms_norm_backward", G.ptr(dg), G.ptr(dw), G.ptr(dx), G.ptr(dr), G.ptr(gx), G.ptr(gt), rows, cols)
+    norm, got_rms = G.dev(np.full(offset + rows * cols + guard, 7.0, np.float32)), G.dev(np.full(rows + guard, 7.0, np.float32))
+    _call("pxk_rms_norm_forward", G.ptr(dx), G.ptr(dw), G.ptr(norm[offset:]), G.ptr(got_rms), rows, cols, ctypes.c_float(1e-5))
+    outs += [norm, got_rms]
     for o in outs + [lse]:
         assert np.all(G.host(o)[-guard:] == 7.0)
     host = lambda o: G.host(o)[:rows * cols].reshape(rows, cols).astype(np.float64)  # noqa: E731
     assert np.all(np.abs(host(p) - P) <= 2e-6 * P)
     want = X.max(1) + np.log(E.sum(1))
     assert np.all(np.abs(G.host(lse)[:rows] - want) <= 1e-6 * (1.0 + np.abs(want)))
+    want = np.sqrt((X ** 2).mean(1) + 1e-5)
+    assert np.all(np.abs(G.host(got_rms)[:rows] - want) <= 1e-6 * want)
+    assert np.all(np.abs(host(norm[offset:]) - W * X / want[:, None]) <= 1e-6 * np.abs(W * X / want[:, None]))
     dot, size = (X * Gr).sum(1, keepdims=True), np.abs(X * Gr).sum(1, keepdims=True)
     assert np.all(np.abs(host(dp) - X * (Gr - dot)) <= 1e-6 * np.abs(X) * (np.abs(Gr) + size))
     Rc = R[:, None]
