@@ -379,6 +379,107 @@ __global__ void __launch_bounds__(kThreads) attention_lrp_scores_kernel(const fl
     }
 }
 
+// Both for sequences of up to 64 NV keys, where a wave that walks a row waits out the memory latency of
+// every 64 keys of it, in three passes and two: lane j holds keys j, j + 64, ... in registers, their
+// loads in flight together, and sums them in the order of the walk, so the results are the same to the
+// bit. (Loads past the visible keys are not issued: their memory may never have been written.)
+// 9 heads of 3072 keys, walked and held: softmax 214 and 149 us, scores 191 and 146. For the spans that
+// were measured, past 2048 keys up to what 64 registers hold.
+constexpr int kHeldKeys = 64;
+
+template <int NV>
+__global__ void __launch_bounds__(kThreads) attention_softmax_held_kernel(const float* raw, float* p, int64_t rows,
+                                                                          int64_t L, float scale, int causal,
+                                                                          int64_t window) {
+    const int64_t r = row_id();
+    if (r >= rows) return;
+    const int lane = lane_id();
+    int64_t lo64, vis64;
+    visible_keys(r % L, L, causal, window, lo64, vis64);
+    const int lo = static_cast<int>(lo64), vis = static_cast<int>(vis64), len = static_cast<int>(L);
+    const float* x = raw + r * L;
+    float v[NV];
+#pragma unroll
+    for (int b = 0; b < NV; b += 8) {  // key lo + lane + 64 i, as the walk takes them
+        const bool any = lo + kWave * b < vis;  // uniform
+#pragma unroll
+        for (int i = b; i < b + 8; ++i) {
+            const int j = lo + lane + kWave * i;
+            v[i] = any ? x[j < vis ? j : vis - 1] : 0.0f;
+        }
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+        if (lo + lane + kWave * i < vis) mx = fmaxf(mx, scale * v[i]);
+    mx = wave_max(mx);
+    float s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+        if (lo + lane + kWave * i < vis) {
+            v[i] = expf(fmaf(scale, v[i], -mx));  // as the walk's expression contracts
+            s += v[i];
+        }
+    s = wave_sum(s);
+    float* y = p + r * L;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int j = lo + lane + kWave * i;
+        if (j < vis) y[j] = v[i] / s;
+    }
+    for (int j = lane; j < lo; j += kWave) y[j] = 0.0f;
+    for (int j = vis + lane; j < len; j += kWave) y[j] = 0.0f;
+}
+
+template <int NV>
+__global__ void __launch_bounds__(kThreads) attention_lrp_scores_held_kernel(const float* r_attn, const float* p,
+                                                                             const float* raw, float* s_out,
+                                                                             int64_t rows, int64_t L, float scale,
+                                                                             float eps, int causal, int64_t window) {
+    constexpr int STEP = 8;  // P and raw vectors in flight
+    const int64_t r = row_id();
+    if (r >= rows) return;
+    const int lane = lane_id();
+    int64_t lo64, vis64;
+    visible_keys(r % L, L, causal, window, lo64, vis64);
+    const int lo = static_cast<int>(lo64), vis = static_cast<int>(vis64), len = static_cast<int>(L);
+    const int64_t off = r * L;
+    float v[NV];
+#pragma unroll
+    for (int b = 0; b < NV; b += 8) {
+        const bool any = lo + kWave * b < vis;  // uniform
+#pragma unroll
+        for (int i = b; i < b + 8; ++i) {
+            const int j = lo + lane + kWave * i;
+            v[i] = any ? r_attn[off + (j < vis ? j : vis - 1)] : 0.0f;
+        }
+    }
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+        if (lo + lane + kWave * i < vis) sum += v[i];
+    sum = wave_sum(sum);
+#pragma unroll
+    for (int b = 0; b < NV; b += STEP) {
+        if (lo + kWave * b >= vis) break;  // uniform
+        float pv[STEP], o[STEP];
+#pragma unroll
+        for (int u = 0; u < STEP; ++u) {
+            const int j = lo + lane + kWave * (b + u), jj = j < vis ? j : vis - 1;
+            pv[u] = p[off + jj];
+            o[u] = raw[off + jj];
+        }
+#pragma unroll
+        for (int u = 0; u < STEP; ++u) {
+            const int j = lo + lane + kWave * (b + u);
+            const float rs = (scale * o[u]) * (v[b + u] - pv[u] * sum);
+            if (j < vis) s_out[off + j] = rs / (2.0f * o[u] + eps * ((o[u] >= 0.0f) ? 1.0f : -1.0f));
+        }
+    }
+    for (int j = lane; j < lo; j += kWave) s_out[off + j] = 0.0f;
+    for (int j = vis + lane; j < len; j += kWave) s_out[off + j] = 0.0f;
+}
+
 // RMSNorm over each head's D values of head-packed rows (QK-Norm, multihead_attention_module.cpp
 // step 3): wave per (row, head); in row m, head h at in + m * ld_in + h * D.
 __global__ void __launch_bounds__(kThreads) rms_norm_heads_kernel(const float* in, int64_t ld_in, float* out,
@@ -800,8 +901,13 @@ int pxk_attention_softmax(const float* raw, float* p, int64_t slices, int64_t l,
     int rc;
     if (!sizes_ok("pxk_attention_softmax", slices, l, &rc)) return rc;
     if (window < 0) return fail(PXK_ERR_INVALID, "pxk_attention_softmax: negative window");
-    PXK_LAUNCH(attention_softmax_kernel, dim3(rows_grid(slices * l)), dim3(kThreads), 0, S(stream), raw, p,
-                       slices * l, l, scale, causal, window);
+    const int64_t span = causal && window > 0 && window < l ? window : l;
+    const dim3 grid(rows_grid(slices * l)), block(kThreads);
+    if (span > 2048 && span <= 64 * kHeldKeys && l <= (int64_t{1} << 30))
+        PXK_LAUNCH(attention_softmax_held_kernel<kHeldKeys>, grid, block, 0, S(stream), raw, p, slices * l, l, scale,
+                   causal, window);
+    else
+        PXK_LAUNCH(attention_softmax_kernel, grid, block, 0, S(stream), raw, p, slices * l, l, scale, causal, window);
     return launched("pxk_attention_softmax");
 }
 
@@ -810,8 +916,14 @@ int pxk_attention_lrp_scores(const float* r_attn, const float* p, const float* r
     int rc;
     if (!sizes_ok("pxk_attention_lrp_scores", slices, l, &rc)) return rc;
     if (window < 0) return fail(PXK_ERR_INVALID, "pxk_attention_lrp_scores: negative window");
-    PXK_LAUNCH(attention_lrp_scores_kernel, dim3(rows_grid(slices * l)), dim3(kThreads), 0, S(stream), r_attn,
-                       p, raw, s, slices * l, l, scale, eps, causal, window);
+    const int64_t span = causal && window > 0 && window < l ? window : l;
+    const dim3 grid(rows_grid(slices * l)), block(kThreads);
+    if (span > 2048 && span <= 64 * kHeldKeys && l <= (int64_t{1} << 30))  // as pxk_attention_softmax
+        PXK_LAUNCH(attention_lrp_scores_held_kernel<kHeldKeys>, grid, block, 0, S(stream), r_attn, p, raw, s, slices * l,
+                   l, scale, eps, causal, window);
+    else
+        PXK_LAUNCH(attention_lrp_scores_kernel, grid, block, 0, S(stream), r_attn, p, raw, s, slices * l, l, scale, eps,
+                   causal, window);
     return launched("pxk_attention_lrp_scores");
 }
 
