@@ -135,8 +135,10 @@ enum {
                              to about 4000 rows at m <= 4). PXK_TILE_AUTO picks it whenever it applies */
     PXK_TILE_32x48_DIRECT = 8, /* as 32x64 direct, 48 columns: 192 workgroups over a 512 x 576 output */
     PXK_TILE_32x48 = 9,       /* as 32x64, 48 columns */
-    /* fp32 products on the bf16 matrix units, every operand split exactly into three bf16 parts
-     * (fp32 accumulation; no less exact than the fp32 MFMA, gemm_impl.hpp) */
+    /* fp32 products on the bf16 matrix units, every finite operand split exactly into three bf16 parts
+     * (fp32 accumulation; no less exact than the fp32 MFMA, gemm_impl.hpp). An output tile with a result
+     * above 2^79, or that reads an element above 2^103, an infinity or NaN, runs on the fp32 MFMA, at
+     * about three times its time */
     PXK_TILE_128x128_SPLIT = 10,
     PXK_TILE_64x64_SPLIT = 11
 };

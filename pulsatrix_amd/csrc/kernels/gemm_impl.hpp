@@ -1315,29 +1315,36 @@ __global__ void __launch_bounds__(NT) skinny_nt_kernel(const Args g) {
 }
 
 // ---- split-bf16 tiles -----------------------------------------------------------------------------
-// The fp32 product on the bf16 matrix units. Each operand element is split exactly into three bf16
-// parts, x = h + m + l (each the round-to-nearest of what is left: 8 + 8 + 8 significant bits and the
-// signs between them hold fp32's 24), and A B is summed as hh + (hm + mh + mm + hl + lh) with
+// The fp32 product on the bf16 matrix units. Each operand element, scaled by 2^24, is split into three
+// bf16 parts, x = h + m + l (each the round-to-nearest of what is left: 8 + 8 + 8 significant bits and
+// the signs between them hold fp32's 24), and A B is summed as hh + (hm + mh + mm + hl + lh) with
 // v_mfma_f32_16x16x32_bf16: six products at 16 times the fp32 MFMA's rate, 2.67x its throughput. The
-// terms left out (ml, lm, ll) are below 2^-25 of a product; each part's product is exact in the fp32
-// accumulator, which rounds to nearest. hh has an accumulator of its own and the five small terms
-// another, so the large sum is rounded once per 32 K steps instead of once per 4: measured against
+// scale makes the split exact for every |x| below 2^103: the last bit of fp32's least subnormal, 2^-149,
+// becomes 2^-125, and every part is zero or a normal bf16 number. (Without it the low parts of elements
+// below 2^-110 are lost, whatever they are multiplied by.) It costs a multiplication an element, 1-5% of
+// a launch. The terms left out (ml, lm, ll) are below 2^-25 of a product; each part's product is exact in
+// the fp32 accumulator, which rounds to nearest. hh has an accumulator of its own and the five small
+// terms another, so the large sum is rounded once per 32 K steps instead of once per 4: measured against
 // float64 over normal, positive and 4-sigma log-normal operands, the error is 0.3-1.0 of the fp32
 // MFMA's at K = 64 .. 8192 (relative 2-norm 4.3e-7 -> 1.4e-7 at K = 576, 1.6e-6 -> 5.7e-7 at 8192).
-// Infinities, NaN, overflow and results below 2^-90 (whose operands' low parts may lie under bf16's
-// subnormals) are not left to the split: a tile with any such element is computed again on the fp32
-// MFMA, so they come out as they always did.
+//
+// What overflows on the way (a result above 2^79, an element above 2^103, infinities, NaN) ends as an
+// infinity or NaN: a tile with any such result is computed again on the fp32 MFMA from memory, so that
+// it comes out as the fp32 tiles give it. Such a tile costs about three times its time: a 128x128
+// launch of 2048^3 with one, 127 -> 285 us, and all of 8192 x 2048 x 2048, 346 -> 970 (the fp32 tile 504).
 //
 // A stage of BK = 32 KS is loaded to registers as fp32 (one stage ahead), split once per element on its
-// way to LDS, and read back as ready MFMA fragments. LDS holds, per operand and part, 16-byte pieces of eight K values (4 q .. 4 q + 3 and 16 + 4 q .. of a 32-deep slice, so that the
-// loads of a row are contiguous across lanes; A and B agree on the order), placed free of bank
-// conflicts (SplitPanel::place).
+// way to LDS, and read back as ready MFMA fragments. LDS holds, per operand and part, 16-byte pieces of
+// eight K values (4 q .. 4 q + 3 and 16 + 4 q .. of a 32-deep slice, so that the loads of a row are
+// contiguous across lanes; A and B agree on the order), placed free of bank conflicts
+// (SplitPanel::place).
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
 typedef float f2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
-constexpr float kSplitTiny = 8.077935669463161e-28f;  // 2^-90
+constexpr float kSplitScale = 16777216.0f;              // 2^24, of A and of B
+constexpr float kSplitUnscale = 3.552713678800501e-15f;  // 2^-48
 
 // Two floats to a packed bf16 pair (round to nearest even), and what is left of each.
 __device__ __forceinline__ uint32_t bf16_pair(float& a, float& b) {
@@ -1347,6 +1354,8 @@ __device__ __forceinline__ uint32_t bf16_pair(float& a, float& b) {
     return p;
 }
 __device__ __forceinline__ void split8(float (&x)[8], u4 (&part)[3]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] *= kSplitScale;
 #pragma unroll
     for (int p = 0; p < 3; ++p)
 #pragma unroll
@@ -1490,16 +1499,18 @@ struct SplitPanel {
     }
 };
 
-// The tile on the fp32 MFMA, straight from memory: for the tiles the split does not settle.
+// The tile on the fp32 MFMA, straight from memory, a stage in flight at a time: for the tiles the split
+// does not settle.
 template <class C, bool TA, bool TB, int PRO>
 __device__ __forceinline__ void fp32_tile(const Args& g, f4 (&acc)[C::TM][C::TN], int64_t m0, int64_t n0, int64_t b,
                                           int64_t k_lo, int nkb, int t0, int t1, int ks, int lane) {
     constexpr bool DS = PRO == PXK_PRO_DIV_STAB || PRO == kProStabBias;
-    const int c = lane & 15, kl = lane >> 4;
 #pragma unroll
     for (int i = 0; i < C::TM; ++i)
 #pragma unroll
         for (int j = 0; j < C::TN; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+    float ss[C::TM] = {};  // the rows' sums of squares (PXK_PRO_RMS) are those of the split
+#pragma unroll 1
     for (int t = t0; t < t1; ++t) {
         const int grp = t / nkb;
         const float* A = obase(g.a, b, g.inner, grp);
@@ -1507,29 +1518,16 @@ __device__ __forceinline__ void fp32_tile(const Args& g, f4 (&acc)[C::TM][C::TN]
         const float* Z = DS ? obase(g.z, b, g.inner, grp) : nullptr;
         const float* ZB = PRO == kProStabBias ? obase(g.zb, b, g.inner, grp) : nullptr;
         const int64_t k0 = k_lo + static_cast<int64_t>(t - grp * nkb) * C::BK + 32 * ks;
-#pragma unroll 1
-        for (int kk = kl; kk < 32; kk += 4) {
-            const int64_t k = k0 + kk;
-            float a[C::TM], bb[C::TN];
-#pragma unroll
-            for (int i = 0; i < C::TM; ++i) {
-                const int64_t m = min(m0 + 16 * i + c, g.M - 1);
-                a[i] = k < g.K ? (TA ? A[k * g.a.ld + m] : A[m * g.a.ld + k]) : 0.0f;
-                if constexpr (DS) {
-                    const float z = k < g.K ? (TA ? Z[k * g.z.ld + m] : Z[m * g.z.ld + k]) : 1.0f;
-                    a[i] *= __builtin_amdgcn_rcpf(stab(ZB && k < g.K ? z + ZB[k] : z, g.eps));
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < C::TN; ++j) {
-                const int64_t n = min(n0 + 16 * j + c, g.N - 1);
-                bb[j] = k < g.K ? (TB ? B[n * g.b.ld + k] : B[k * g.b.ld + n]) : 0.0f;
-            }
-#pragma unroll
-            for (int i = 0; i < C::TM; ++i)
-#pragma unroll
-                for (int j = 0; j < C::TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], bb[j], acc[i][j], 0, 0, 0);
+        DirectChunk<C, TA, TB, PRO> ch[2];  // 16 deep each
+        if (k0 + 32 <= g.K) {
+            ch[0].template load<true>(g, A, Z, ZB, B, m0, n0, k0, lane);
+            ch[1].template load<true>(g, A, Z, ZB, B, m0, n0, k0 + 16, lane);
+        } else {
+            ch[0].load_guarded(g, A, Z, ZB, B, m0, n0, k0, lane);
+            ch[1].load_guarded(g, A, Z, ZB, B, m0, n0, k0 + 16, lane);
         }
+        ch[0].mma(acc, g.eps, ss);
+        ch[1].mma(acc, g.eps, ss);
     }
 }
 
@@ -1701,12 +1699,9 @@ __global__ void __launch_bounds__(C::NT, 2) gemm_split_kernel(const Args g) {
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            acc[i][j] += low[i][j];
+            acc[i][j] = (acc[i][j] + low[i][j]) * kSplitUnscale;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float v = fabsf(acc[i][j][r]);
-                redo |= !(v <= 3.4028234663852886e38f) || (v < kSplitTiny && v != 0.0f);
-            }
+            for (int r = 0; r < 4; ++r) redo |= !(fabsf(acc[i][j][r]) <= 3.4028234663852886e38f);
         }
     if (__syncthreads_or(redo))
         fp32_tile<C, TA, TB, PRO>(g, acc, m0 + wm, n0 + wn, b, k_lo, nkb, t0, t1, ks, lane);

@@ -78,6 +78,33 @@ def test_values_the_split_cannot_hold(tile, splits):
 
 @gpu
 @pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("where", ["a", "b"])
+@pytest.mark.parametrize("small,large", [(3e-31, 1e8), (1e-33, 1e10), (1e-36, 1e20), (1e-38, 1e25), (1e-41, 1e30), (1e-21, 1e-21)])
+def test_small_operands(tile, where, small, large):
+    """A row of A (a column of B) whose bf16 parts would be subnormal or nothing, against a large other
+    operand: no result of the tile is small, and all are as exact as the fp32 tiles give them (subnormal
+    ones, of 1e-21 by 1e-21, to their last bits)."""
+    rng = np.random.RandomState(11)
+    a, b = rng.standard_normal((130, 96)).astype(np.float32), rng.standard_normal((96, 70)).astype(np.float32)
+    if where == "a":
+        a[129] *= np.float32(small)
+        b *= np.float32(large)
+    else:
+        b[:, 2] *= np.float32(small)
+        a *= np.float32(large)
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    size = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)
+    # 24 fp32 MFMAs of four K steps each round their running sum, which stays below size, by at most 2^-24
+    # of it (half of that on average); subnormal products are off by 2^-149 each
+    bound = 12 * 2.0 ** -24 * size + 96 * 2.0 ** -149
+    for t in (tile, N.TILE_64x64):
+        off = np.abs(product(a, b, 0, 0, t) - want) / bound
+        print("tile %d: at most %.3g of the bound" % (t, off.max()))
+        assert off.max() <= 1.0
+
+
+@gpu
+@pytest.mark.parametrize("tile", TILES)
 def test_no_less_exact_than_the_fp32_tiles(tile):
     """Against float64 on normal, positive and heavy-tailed operands, beside the fp32 MFMA's direct tile. The
     split tiles stand where one fp32 accumulator ran over the whole of K; the direct tile adds four
