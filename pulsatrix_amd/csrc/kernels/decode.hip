@@ -330,17 +330,19 @@ __global__ void __launch_bounds__(kThreads) decode_attention_merge_kernel(const 
             const float m = tid < nc ? part[tid * ps] : -INFINITY;
             mass[tid] = tid < nc ? part[tid * ps + 1] : 0.0f;
             const float M = wave_max(m);
-            weight[tid] = m != -INFINITY ? expf(m - M) : 0.0f;  // an empty chunk's partial is zeros
+            weight[tid] = m != -INFINITY ? expf(m - M) : -1.0f;  // -1: counts for nothing, whatever its partial
         }
         __syncthreads();
         float l = 0.0f;
-        for (int c = 0; c < nc; ++c) l += weight[c] * mass[c];
+        for (int c = 0; c < nc; ++c)
+            if (!(weight[c] < 0.0f)) l += weight[c] * mass[c];
         for (int64_t d = tid; d < a.D; d += kThreads) {
             float acc = 0.0f;
 #pragma unroll
             for (int c = 0; c < kAhead; ++c)
-                if (c < nc) acc += weight[c] * (d == tid ? ahead[c] : part[c * ps + kPartHead + d]);
-            for (int c = kAhead; c < nc; ++c) acc += weight[c] * part[c * ps + kPartHead + d];
+                if (c < nc && !(weight[c] < 0.0f)) acc += weight[c] * (d == tid ? ahead[c] : part[c * ps + kPartHead + d]);
+            for (int c = kAhead; c < nc; ++c)
+                if (!(weight[c] < 0.0f)) acc += weight[c] * part[c * ps + kPartHead + d];
             a.ctx[bh * a.D + d] = acc / l;
         }
         return;

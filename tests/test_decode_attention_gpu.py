@@ -8,11 +8,15 @@ import gpu_util as G
 from pulsatrix_amd import native as N
 
 
-def run(n, H, Hkv, D, cap, pos, window):
+def run(n, H, Hkv, D, cap, pos, window, masked=()):
+    """masked: keys of every sequence whose scores are all -inf."""
     rng = np.random.RandomState(D + pos)
     q = rng.standard_normal((n, H, D)).astype(np.float32)
     k, v = (rng.standard_normal((n, cap, Hkv, D)).astype(np.float32) for _ in range(2))
     k[:, pos + 1:], v[:, pos + 1:] = np.nan, np.nan
+    if len(masked):
+        q[..., 0] = np.abs(q[..., 0]) + 1.0
+        k[:, list(masked), :, 0] = -np.inf
     lo = max(0, pos + 1 - window) if window else 0
     torch = G.torch_cuda()
     dq, dk, dv, ctx = G.dev(q), G.dev(k), G.dev(v), G.empty((n, H, D))
@@ -44,6 +48,15 @@ def test_head_dims_and_positions(D, pos):
 @pytest.mark.parametrize("pos,window", [(5, 1), (70, 7), (100, 64), (130, 65), (130, 200)])
 def test_windows(D, pos, window):
     run(3, 2, 1, D, 140, pos, window)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [6, 40, 64, 256, 320])
+@pytest.mark.parametrize("cap,pos,masked", [(131, 130, range(64)), (131, 130, range(3, 64)), (300, 299, range(64, 192)), (300, 299, range(192, 299)),
+                                            (70, 69, range(64, 70)), (4160, 4159, range(128, 256))])
+def test_chunks_of_scores_minus_infinity(cap, pos, masked, D):
+    """A chunk whose every score is -inf counts for nothing, like one that holds no key."""
+    run(2, 2, 1, D, cap, pos, 0, masked)
 
 
 @pytest.mark.gpu
