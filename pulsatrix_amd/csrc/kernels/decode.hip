@@ -333,16 +333,18 @@ __global__ void __launch_bounds__(kThreads) decode_attention_merge_kernel(const 
             weight[tid] = m != -INFINITY ? expf(m - M) : -1.0f;  // -1: counts for nothing, whatever its partial
         }
         __syncthreads();
+        auto weighed = [&](int c, float x) {  // selects, no branches: the loads below issue back to back
+            const float w = weight[c];
+            return w < 0.0f ? 0.0f : w * x;
+        };
         float l = 0.0f;
-        for (int c = 0; c < nc; ++c)
-            if (!(weight[c] < 0.0f)) l += weight[c] * mass[c];
+        for (int c = 0; c < nc; ++c) l += weighed(c, mass[c]);
         for (int64_t d = tid; d < a.D; d += kThreads) {
             float acc = 0.0f;
 #pragma unroll
             for (int c = 0; c < kAhead; ++c)
-                if (c < nc && !(weight[c] < 0.0f)) acc += weight[c] * (d == tid ? ahead[c] : part[c * ps + kPartHead + d]);
-            for (int c = kAhead; c < nc; ++c)
-                if (!(weight[c] < 0.0f)) acc += weight[c] * part[c * ps + kPartHead + d];
+                if (c < nc) acc += weighed(c, d == tid ? ahead[c] : part[c * ps + kPartHead + d]);
+            for (int c = kAhead; c < nc; ++c) acc += weighed(c, part[c * ps + kPartHead + d]);
             a.ctx[bh * a.D + d] = acc / l;
         }
         return;
