@@ -313,42 +313,47 @@ __global__ void __launch_bounds__(kThreads) decode_attention_part_vec_kernel(con
 }
 
 // Second pass, one workgroup per (sequence, query head): the chunks' partials merged with their
-// maxima, ctx = sum_c e^(m_c - M) acc_c / sum_c e^(m_c - M) l_c.
+// maxima, ctx = sum_c e^(m_c - M) acc_c / sum_c e^(m_c - M) l_c. A chunk whose maximum is -inf counts
+// for nothing, whatever its partial. This form for up to kWave chunks (4096 positions): every chunk's
+// weight at once, a lane each; at 64 chunks 7 us where the walk below takes 43.
+__global__ void __launch_bounds__(kThreads) decode_attention_merge_few_kernel(const DecodeAttnArgs a) {
+    __shared__ float weight[kWave], mass[kWave];
+    constexpr int kAhead = 4;  // partials in flight beside the maxima
+    const int64_t bh = blockIdx.x;
+    const int64_t ps = a.D + kPartHead;
+    const float* part = a.part + bh * a.chunks * ps;
+    const int tid = threadIdx.x, nc = static_cast<int>(a.chunks);
+    const float* col = part + kPartHead + (tid < a.D ? tid : a.D - 1);
+    float ahead[kAhead];
+#pragma unroll
+    for (int c = 0; c < kAhead; ++c) ahead[c] = col[min(c, nc - 1) * ps];
+    if (tid < kWave) {
+        const float m = tid < nc ? part[tid * ps] : -INFINITY;
+        mass[tid] = tid < nc ? part[tid * ps + 1] : 0.0f;
+        const float M = wave_max(m);
+        weight[tid] = m != -INFINITY ? expf(m - M) : -1.0f;  // -1: counts for nothing
+    }
+    __syncthreads();
+    auto weighed = [&](int c, float x) {  // selects, no branches: the loads below issue back to back
+        const float w = weight[c];
+        return w < 0.0f ? 0.0f : w * x;
+    };
+    float l = 0.0f;
+    for (int c = 0; c < nc; ++c) l += weighed(c, mass[c]);
+    for (int64_t d = tid; d < a.D; d += kThreads) {
+        float acc = 0.0f;
+#pragma unroll
+        for (int c = 0; c < kAhead; ++c)
+            if (c < nc) acc += weighed(c, d == tid ? ahead[c] : part[c * ps + kPartHead + d]);
+        for (int c = kAhead; c < nc; ++c) acc += weighed(c, part[c * ps + kPartHead + d]);
+        a.ctx[bh * a.D + d] = acc / l;
+    }
+}
+
 __global__ void __launch_bounds__(kThreads) decode_attention_merge_kernel(const DecodeAttnArgs a) {
     const int64_t bh = blockIdx.x;
     const int64_t ps = a.D + kPartHead;
     const float* part = a.part + bh * a.chunks * ps;
-    if (a.chunks <= kWave) {  // up to 4096 positions: every chunk's weight at once, a lane each
-        __shared__ float weight[kWave], mass[kWave];
-        constexpr int kAhead = 4;  // partials in flight beside the maxima
-        const int tid = threadIdx.x, nc = static_cast<int>(a.chunks);
-        const float* col = part + kPartHead + (tid < a.D ? tid : a.D - 1);
-        float ahead[kAhead];
-#pragma unroll
-        for (int c = 0; c < kAhead; ++c) ahead[c] = col[min(c, nc - 1) * ps];
-        if (tid < kWave) {
-            const float m = tid < nc ? part[tid * ps] : -INFINITY;
-            mass[tid] = tid < nc ? part[tid * ps + 1] : 0.0f;
-            const float M = wave_max(m);
-            weight[tid] = m != -INFINITY ? expf(m - M) : -1.0f;  // -1: counts for nothing, whatever its partial
-        }
-        __syncthreads();
-        auto weighed = [&](int c, float x) {  // selects, no branches: the loads below issue back to back
-            const float w = weight[c];
-            return w < 0.0f ? 0.0f : w * x;
-        };
-        float l = 0.0f;
-        for (int c = 0; c < nc; ++c) l += weighed(c, mass[c]);
-        for (int64_t d = tid; d < a.D; d += kThreads) {
-            float acc = 0.0f;
-#pragma unroll
-            for (int c = 0; c < kAhead; ++c)
-                if (c < nc) acc += weighed(c, d == tid ? ahead[c] : part[c * ps + kPartHead + d]);
-            for (int c = kAhead; c < nc; ++c) acc += weighed(c, part[c * ps + kPartHead + d]);
-            a.ctx[bh * a.D + d] = acc / l;
-        }
-        return;
-    }
     float M = -INFINITY;
     for (int64_t c = 0; c < a.chunks; ++c) M = fmaxf(M, part[c * ps]);
     float l = 0.0f;
@@ -554,8 +559,12 @@ extern "C" int pxk_decode_attention(const float* q, const float* k_cache, const 
     else
         PXK_LAUNCH(decode_attention_part_kernel, grid, dim3(kThreads), lds, S(stream), a);
     if (const int rc = launched("pxk_decode_attention")) return rc;
-    PXK_LAUNCH(decode_attention_merge_kernel, dim3(static_cast<unsigned>(n * heads)), dim3(kThreads), 0,
-                       S(stream), a);
+    if (chunks <= kWave)
+        PXK_LAUNCH(decode_attention_merge_few_kernel, dim3(static_cast<unsigned>(n * heads)), dim3(kThreads), 0,
+                   S(stream), a);
+    else
+        PXK_LAUNCH(decode_attention_merge_kernel, dim3(static_cast<unsigned>(n * heads)), dim3(kThreads), 0,
+                   S(stream), a);
     return launched("pxk_decode_attention (merge)");
 }
 
