@@ -549,12 +549,16 @@ extern "C" int pxk_decode_attention(const float* q, const float* k_cache, const 
     const DecodeAttnArgs a{q,        k_cache, v_cache,  seq_stride, ctx,   workspace, pos, heads,
                            kv_heads, head_dim, window, max_keys, chunks, scale, vec};
     const dim3 grid(static_cast<unsigned>(n * heads * chunks));
-    // A thread holds head_dim / 16 vectors of K and of V; past 256 they are read in loops.
+    // A thread holds head_dim / 16 vectors of K and of V; past 256 they are read in loops. So they are past
+    // 128 where more than 512 workgroups (two a CU) share the chip: 128 held floats leave a SIMD two
+    // waves, and other workgroups hide the latency that holding them would. Caches cold, in loops and held:
+    // 8 heads of 256, 256 workgroups 15.1 and 11.2 us, 512 18.6 and 16.8, 1024 28.1 and 27.7, 8192 158 and
+    // 177; with K and V in L2 1024 13.8 and 17.0, 8192 117 and 151.
     if (vec && head_dim <= 64)
         PXK_LAUNCH(decode_attention_part_vec_kernel<4>, grid, dim3(kThreads), 0, S(stream), a);
     else if (vec && head_dim <= 128)
         PXK_LAUNCH(decode_attention_part_vec_kernel<8>, grid, dim3(kThreads), 0, S(stream), a);
-    else if (vec && head_dim <= 256)
+    else if (vec && head_dim <= 256 && n * heads * chunks <= 512)
         PXK_LAUNCH(decode_attention_part_vec_kernel<16>, grid, dim3(kThreads), 0, S(stream), a);
     else
         PXK_LAUNCH(decode_attention_part_kernel, grid, dim3(kThreads), lds, S(stream), a);
