@@ -383,8 +383,11 @@ __global__ void __launch_bounds__(kThreads) attention_lrp_scores_kernel(const fl
 // every 64 keys of it, in three passes and two: lane j holds keys j, j + 64, ... in registers, their
 // loads in flight together, and sums them in the order of the walk, so the results are the same to the
 // bit. (Loads past the visible keys are not issued: their memory may never have been written.)
-// 9 heads of 3072 keys, walked and held: softmax 214 and 149 us, scores 191 and 146. For the spans that
-// were measured, past 2048 keys up to what 64 registers hold.
+// Past 2048 keys, up to what 64 registers hold; measured at 2049 .. 4096 keys of 1 to 32 heads, causal and
+// not, and with windows of 2100 and 4000: the softmax takes 0.34-0.76 of the walk's time, the scores
+// 0.45-0.92 (9 causal heads, walked and held: 2049 keys 72 and 42 us, 103 and 75; 3072 224 and 101, 203
+// and 163; 4096 383 and 165, 350 and 278). Blocks of 512 keys that a row does not reach are skipped whole:
+// computed and dropped, they made the softmax slower than the walk up to 2304 keys (72 against 87 us).
 constexpr int kHeldKeys = 64;
 
 template <int NV>
@@ -410,22 +413,34 @@ __global__ void __launch_bounds__(kThreads) attention_softmax_held_kernel(const 
     }
     float mx = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
-        if (lo + lane + kWave * i < vis) mx = fmaxf(mx, scale * v[i]);
+    for (int b = 0; b < NV; b += 8) {
+        if (lo + kWave * b >= vis) break;  // uniform
+#pragma unroll
+        for (int i = b; i < b + 8; ++i)
+            if (lo + lane + kWave * i < vis) mx = fmaxf(mx, scale * v[i]);
+    }
     mx = wave_max(mx);
     float s = 0.0f;
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
-        if (lo + lane + kWave * i < vis) {
-            v[i] = expf(fmaf(scale, v[i], -mx));  // as the walk's expression contracts
-            s += v[i];
-        }
+    for (int b = 0; b < NV; b += 8) {
+        if (lo + kWave * b >= vis) break;
+#pragma unroll
+        for (int i = b; i < b + 8; ++i)
+            if (lo + lane + kWave * i < vis) {
+                v[i] = expf(fmaf(scale, v[i], -mx));  // as the walk's expression contracts
+                s += v[i];
+            }
+    }
     s = wave_sum(s);
     float* y = p + r * L;
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        const int j = lo + lane + kWave * i;
-        if (j < vis) y[j] = v[i] / s;
+    for (int b = 0; b < NV; b += 8) {
+        if (lo + kWave * b >= vis) break;
+#pragma unroll
+        for (int i = b; i < b + 8; ++i) {
+            const int j = lo + lane + kWave * i;
+            if (j < vis) y[j] = v[i] / s;
+        }
     }
     for (int j = lane; j < lo; j += kWave) y[j] = 0.0f;
     for (int j = vis + lane; j < len; j += kWave) y[j] = 0.0f;
@@ -456,8 +471,12 @@ __global__ void __launch_bounds__(kThreads) attention_lrp_scores_held_kernel(con
     }
     float sum = 0.0f;
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
-        if (lo + lane + kWave * i < vis) sum += v[i];
+    for (int b = 0; b < NV; b += 8) {
+        if (lo + kWave * b >= vis) break;  // uniform
+#pragma unroll
+        for (int i = b; i < b + 8; ++i)
+            if (lo + lane + kWave * i < vis) sum += v[i];
+    }
     sum = wave_sum(sum);
 #pragma unroll
     for (int b = 0; b < NV; b += STEP) {
