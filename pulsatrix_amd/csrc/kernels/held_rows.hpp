@@ -24,7 +24,10 @@ struct HeldShape {
 // x 64: 5.5 us, 7.1 held). One wave a row up to 1024 columns, where a workgroup a row would leave most
 // of its threads a float4 or less; above, a workgroup, which keeps a thread's share under 32 floats an
 // operand up to 8192 columns. RMSNorm's backward, walked and held: 16384 x 500 32.6 and 20.4 us, 4096 x
-// 1001 20.7 and 11.4, 2048 x 8191 117 and 47, 8 x 576 5.6 and 3.4, 1 x 4096 27.3 and 3.5.
+// 1001 20.7 and 11.4, 2048 x 8191 117 and 47, 8 x 576 5.6 and 3.4, 1 x 4096 27.3 and 3.5. The single-float
+// shapes are the finer ones: a place that holds no column costs its exponential and store all the same
+// (log-sum-exp, walked and held in twice the places or more: 16384 x 257 9.0 and 10.3 us, 16384 x 2049 51
+// and 63; as below 7.0 and 29).
 template <class F>
 bool with_held_shape(int64_t cols, bool vec, F&& f) {
     if (cols <= kWave) return false;
@@ -38,8 +41,13 @@ bool with_held_shape(int64_t cols, bool vec, F&& f) {
         else return false;
     } else {
         if (cols <= 256) f(HeldShape<64, 1, 4>{});
+        else if (cols <= 512) f(HeldShape<64, 1, 8>{});
         else if (cols <= 1024) f(HeldShape<64, 1, 16>{});
+        else if (cols <= 1536) f(HeldShape<256, 1, 6>{});
         else if (cols <= 2048) f(HeldShape<256, 1, 8>{});
+        else if (cols <= 3072) f(HeldShape<256, 1, 12>{});
+        else if (cols <= 4096) f(HeldShape<256, 1, 16>{});
+        else if (cols <= 6144) f(HeldShape<256, 1, 24>{});
         else if (cols <= 8192) f(HeldShape<256, 1, 32>{});
         else return false;
     }
