@@ -21,7 +21,8 @@ struct HeldShape {
 // Calls f with the shape for rows of `cols` floats; false (f not called) for rows that no shape holds.
 // vec: every operand is 16-byte aligned (a ragged width then still takes single floats). Up to 64
 // columns a row is one step of the walking wave, which loses nothing by it (RMSNorm's backward at 16384
-// x 64: 5.5 us, 7.1 held). One wave a row up to 1024 columns, where a workgroup a row would leave most
+// x 64: 5.5 us, 7.1 held). Up to 128 a float4 a thread would leave half the wave idle (16384 x 128: 7.8 us
+// walked, 8.6 so, 6.5 by single floats). One wave a row up to 1024 columns, where a workgroup a row would leave most
 // of its threads a float4 or less; above, a workgroup, which keeps a thread's share under 32 floats an
 // operand up to 8192 columns. RMSNorm's backward, walked and held: 16384 x 500 32.6 and 20.4 us, 4096 x
 // 1001 20.7 and 11.4, 2048 x 8191 117 and 47, 8 x 576 5.6 and 3.4, 1 x 4096 27.3 and 3.5. The single-float
@@ -31,7 +32,9 @@ struct HeldShape {
 template <class F>
 bool with_held_shape(int64_t cols, bool vec, F&& f) {
     if (cols <= kWave) return false;
-    if (vec && cols % 4 == 0) {
+    if (cols <= 128) {
+        f(HeldShape<64, 1, 2>{});
+    } else if (vec && cols % 4 == 0) {
         if (cols <= 256) f(HeldShape<64, 4, 1>{});
         else if (cols <= 512) f(HeldShape<64, 4, 2>{});
         else if (cols <= 1024) f(HeldShape<64, 4, 4>{});
