@@ -313,7 +313,7 @@ __global__ void __launch_bounds__(kThreads) accumulate_rows_kernel(const float* 
     out[j] = acc;
 }
 
-// Few rows: one thread per column, in row order.
+// Few rows or very many columns: one thread per column, in row order.
 __global__ void __launch_bounds__(kThreads) column_sums_short_kernel(const float* in, float* out, int64_t rows,
                                                                      int64_t cols, float beta) {
     const int64_t j = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
@@ -528,8 +528,11 @@ int pxk_accumulate_rows(const float* in, float* out, int64_t rows, int64_t cols,
 int pxk_column_sums(const float* in, float* out, int64_t rows, int64_t cols, float beta, void* stream) {
     if (rows < 0 || cols < 0) return fail(PXK_ERR_INVALID, "pxk_column_sums: negative size");
     if (cols == 0) return PXK_OK;
-    // Up to a quarter of a step of rows, most row lanes would be idle.
-    if (rows <= kSumRows / 4)
+    // One thread a column where most row lanes would be idle, and where the columns alone fill the chip:
+    // its loads of 1 KiB a wave then beat the 64-byte segments. Per thread and in workgroups of 16 columns:
+    // 64 x 8192 7.4 and 3.3 us, 32 x 49152 4.5 and 5.8, 64 x 49152 7.6 and 6.2, 17 x 262144 3.4 and 29.8,
+    // 256 x 262144 73 and 84, 512 x 262144 218 and 155, 1024 x 524288 520 and 857, 1024 x 2^20 1040 and 1712.
+    if (rows <= kSumRows / 4 || rows * 1024 <= cols || cols >= int64_t{1} << 19)
         PXK_LAUNCH(column_sums_short_kernel, dim3(static_cast<unsigned>(cdiv(cols, kThreads))), dim3(kThreads), 0,
                    S(stream), in, out, rows, cols, beta);
     else
