@@ -29,9 +29,10 @@ struct HeldShape {
 // shapes are the finer ones: a place that holds no column costs its exponential and store all the same
 // (log-sum-exp, walked and held in twice the places or more: 16384 x 257 9.0 and 10.3 us, 16384 x 2049 51
 // and 63; as below 7.0 and 29).
+// A launch has fewer than 2^32 threads: 2^24 rows and more of a workgroup each are left to the walk.
 template <class F>
-bool with_held_shape(int64_t cols, bool vec, F&& f) {
-    if (cols <= kWave) return false;
+bool with_held_shape(int64_t rows, int64_t cols, bool vec, F&& f) {
+    if (cols <= kWave || (cols > 1024 && rows >= (int64_t{1} << 24))) return false;
     if (cols <= 128) {
         f(HeldShape<64, 1, 2>{});
     } else if (vec && cols % 4 == 0) {

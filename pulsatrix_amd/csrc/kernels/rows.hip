@@ -830,7 +830,7 @@ int pxk_rms_norm_forward(const float* in, const float* gamma, float* out, float*
         else
             launch_rms_vec<false>(nv, grid, block, S(stream), in, gamma, out, row_rms, rows, cols4, eps);
     } else {
-        const bool held = with_held_shape(cols, aligned16(in) && aligned16(gamma) && aligned16(out), [&](auto shape) {
+        const bool held = with_held_shape(rows, cols, aligned16(in) && aligned16(gamma) && aligned16(out), [&](auto shape) {
             using Shape = decltype(shape);
             PXK_LAUNCH((rms_norm_held_kernel<Shape>), held_grid<Shape>(rows), dim3(kHeldThreads), 0, S(stream), in, gamma,
                        out, row_rms, rows, cols, eps);
@@ -866,7 +866,7 @@ int pxk_rms_norm_add(const float* x, const float* a, const float* gamma_a, float
 int pxk_softmax_rows(const float* in, float* out, int64_t rows, int64_t cols, void* stream) {
     int rc;
     if (!sizes_ok("pxk_softmax_rows", rows, cols, &rc)) return rc;
-    const bool held = with_held_shape(cols, aligned16(in) && aligned16(out), [&](auto shape) {
+    const bool held = with_held_shape(rows, cols, aligned16(in) && aligned16(out), [&](auto shape) {
         using Shape = decltype(shape);
         PXK_LAUNCH((softmax_held_kernel<Shape>), held_grid<Shape>(rows), dim3(kHeldThreads), 0, S(stream), in, out, rows,
                    cols);

@@ -405,7 +405,7 @@ int pxk_elementwise_backward(int op, const float* x, const float* grad_out, floa
 int pxk_softmax_rows_backward(const float* y, const float* dy, float* dx, int64_t rows, int64_t cols, void* stream) {
     int rc;
     if (bad_rows("pxk_softmax_rows_backward", rows, cols, &rc)) return rc;
-    const bool held = with_held_shape(cols, aligned16(y) && aligned16(dy) && aligned16(dx), [&](auto shape) {
+    const bool held = with_held_shape(rows, cols, aligned16(y) && aligned16(dy) && aligned16(dx), [&](auto shape) {
         using Shape = decltype(shape);
         PXK_LAUNCH((softmax_backward_held_kernel<Shape>), held_grid<Shape>(rows), dim3(kHeldThreads), 0, S(stream), y, dy,
                    dx, rows, cols);
@@ -420,7 +420,7 @@ int pxk_rms_norm_backward(const float* grad_out, const float* gamma, const float
     int rc;
     if (bad_rows("pxk_rms_norm_backward", rows, cols, &rc)) return rc;
     const bool vec = aligned16(grad_out) && aligned16(gamma) && aligned16(in) && aligned16(grad_in) && aligned16(gamma_terms);
-    const bool held = with_held_shape(cols, vec, [&](auto shape) {
+    const bool held = with_held_shape(rows, cols, vec, [&](auto shape) {
         using Shape = decltype(shape);
         PXK_LAUNCH((rms_backward_held_kernel<Shape>), held_grid<Shape>(rows), dim3(kHeldThreads), 0, S(stream), grad_out,
                    gamma, in, row_rms, grad_in, gamma_terms, rows, cols);
@@ -453,7 +453,7 @@ int pxk_logsumexp_rows(const float* in, float* out, int64_t rows, int64_t cols, 
     int rc;
     if (cols == 0 && rows > 0) return fail(PXK_ERR_INVALID, "pxk_logsumexp_rows: empty rows");
     if (bad_rows("pxk_logsumexp_rows", rows, cols, &rc)) return rc;
-    const bool held = with_held_shape(cols, aligned16(in), [&](auto shape) {
+    const bool held = with_held_shape(rows, cols, aligned16(in), [&](auto shape) {
         using Shape = decltype(shape);
         PXK_LAUNCH((logsumexp_held_kernel<Shape>), held_grid<Shape>(rows), dim3(kHeldThreads), 0, S(stream), in, out,
                    rows, cols);

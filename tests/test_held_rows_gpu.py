@@ -90,3 +90,21 @@ def test_held_softmax_extremes(cols):
     np.testing.assert_allclose(G.host(lse), L, rtol=1e-6, atol=1e-6)
     _call("pxk_softmax_rows", G.ptr(d), G.ptr(d), 6, cols)  # in place
     assert np.array_equal(G.host(d).reshape(6, cols), G.host(p), equal_nan=True)
+
+
+@pytest.mark.gpu
+def test_more_rows_than_workgroups():
+    """2^24 rows of more than 1024 columns: one workgroup a row would be a launch of 2^32 threads."""
+    torch = G.torch_cuda()
+    rows, cols = 1 << 24, 1028
+    x, lse = torch.zeros(rows, cols, device="cuda"), torch.empty(rows, device="cuda")
+    some = torch.tensor([0, 1, rows // 2, rows - 2, rows - 1], device="cuda")
+    x[some] = torch.randn(len(some), cols, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    want = x[some].double()
+    _call("pxk_logsumexp_rows", G.ptr(x), G.ptr(lse), rows, cols)
+    _call("pxk_softmax_rows", G.ptr(x), G.ptr(x), rows, cols)
+    assert float((lse[some] - want.logsumexp(1)).abs().max()) <= 1e-5
+    assert float((x[some] / want.softmax(1) - 1).abs().max()) <= 2e-6
+    assert float((lse[2:1000] - float(np.log(cols))).abs().max()) <= 1e-5
+    del x
+    torch.cuda.empty_cache()
