@@ -1,5 +1,6 @@
-"""pxk_column_sums at the edges of its 16-column workgroups and 64-row steps against float64: sums of up
-to 1024 terms a lane in fp32 stay within 1e-6 of the column's absolute sum."""
+"""pxk_column_sums at the edges of its 16-column workgroups and 64-row steps, and of the widths that go to
+one thread a column, against float64: sums of up to 1024 terms a lane in fp32 stay within 1e-6 of the
+column's absolute sum."""
 import numpy as np
 import pytest
 
@@ -9,7 +10,7 @@ from pulsatrix_amd import native as N
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,cols", [(0, 5), (1, 1), (16, 300), (17, 300), (63, 16), (64, 17), (65, 15), (511, 33), (513, 100), (4096, 2048),
-                                       (16384, 31)])
+                                       (16384, 31), (17, 17407), (17, 17408), (18, 17408), (30, (1 << 19) - 1), (513, 1 << 19), (700, (1 << 19) - 1)])
 @pytest.mark.parametrize("beta", [0.0, 0.5])
 def test_column_sums(rows, cols, beta):
     rng = np.random.RandomState(rows + cols)
