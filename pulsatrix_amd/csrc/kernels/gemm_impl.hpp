@@ -1402,14 +1402,14 @@ struct SplitPanel {
         k = 32 * (q / 4) + 4 * (q % 4);
     }
     // The thread's pieces' byte offsets from the stage's first element (KC: row r0, K k0; else row k0,
-    // column 0). Rows past the matrix read its last one: what they compute is never stored.
+    // column r0). Rows past the matrix read its last one: what they compute is never stored.
     __device__ __forceinline__ static void lane_offsets(int64_t ld, int64_t mn, int64_t r0, unsigned (&off)[NV]) {
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             int r, k;
             coords(static_cast<int>(threadIdx.x) + i * T, r, k);
-            const int64_t row = min(r0 + r, mn - 1);
-            off[i] = 4u * static_cast<unsigned>(KC ? (row - r0) * ld + k : k * ld + row);
+            const int64_t row = min(r0 + r, mn - 1) - r0;
+            off[i] = 4u * static_cast<unsigned>(KC ? row * ld + k : k * ld + row);
         }
     }
     __device__ __forceinline__ static void load8(const float* base, int64_t ld, unsigned off, float (&x)[8]) {
@@ -1595,10 +1595,10 @@ __global__ void __launch_bounds__(C::NT, 2) gemm_split_kernel(const Args g) {
     int lt = 0;  // stages issued
     auto issue = [&](auto S) {  // the cursor's stage, wholly inside K, into set S; the cursor stops at the last one
         const int64_t k0 = k_lo + static_cast<int64_t>(kb) * BK;
-        pa[S.value].issue(!TA ? A + m0 * g.a.ld + k0 : A + k0 * g.a.ld, g.a.ld, offa,
+        pa[S.value].issue(!TA ? A + m0 * g.a.ld + k0 : A + k0 * g.a.ld + m0, g.a.ld, offa,
                           kZ ? Z + m0 * g.z.ld + k0 : nullptr, g.z.ld, offz, kZB ? ZB + k0 : nullptr);
         const unsigned none[1] = {0};
-        pb[S.value].issue(TB ? B + n0 * g.b.ld + k0 : B + k0 * g.b.ld, g.b.ld, offb, nullptr, 0, none, nullptr);
+        pb[S.value].issue(TB ? B + n0 * g.b.ld + k0 : B + k0 * g.b.ld + n0, g.b.ld, offb, nullptr, 0, none, nullptr);
         if (++lt < nf) advance();
     };
     auto commit = [&](auto S, int buf) {

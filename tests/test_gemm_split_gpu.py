@@ -104,6 +104,26 @@ def test_small_operands(tile, where, small, large):
 
 
 @gpu
+def test_rows_past_32_bit_offsets():
+    """A sliding window over one long row (A^T with a leading dimension of 1): its rows past 2^30 lie past what
+    the lanes' 32-bit byte offsets reach from the matrix's start."""
+    torch = G.torch_cuda()
+    m, k = (1 << 30) + 70, 40
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    row, b, c = torch.randn(m + k - 1, device="cuda", generator=gen), torch.randn(k, device="cuda", generator=gen), torch.empty(m, device="cuda")
+    d = N.GemmDesc()
+    d.m, d.n, d.k, d.batch, d.inner, d.kgroups, d.trans_a, d.tile, d.splits = m, 1, k, 1, 1, 1, 1, N.TILE_128x128_SPLIT, 1
+    d.a, d.b, d.c = N.operand(row.data_ptr(), 1), N.operand(b.data_ptr(), 1), N.operand(c.data_ptr(), 1)
+    N.gemm(d, G.stream())
+    for at in (0, (1 << 30) - 128, m - 100):
+        x = row[at:at + 100 + k - 1].double()
+        want = x.unfold(0, k, 1) @ b.double()
+        assert float((c[at:at + 100].double() - want).norm()) <= 3e-7 * float(want.norm())
+    del row, c
+    torch.cuda.empty_cache()
+
+
+@gpu
 @pytest.mark.parametrize("tile", TILES)
 def test_no_less_exact_than_the_fp32_tiles(tile):
     """Against float64 on normal, positive and heavy-tailed operands, beside the fp32 MFMA's direct tile. The
