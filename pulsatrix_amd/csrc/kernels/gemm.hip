@@ -465,7 +465,8 @@ extern "C" int pxk_gemm(const pxk_gemm_desc* d, void* stream) {
     const int has_bias = d->prologue == PXK_PRO_DIV_STAB && d->z_bias.ptr != nullptr;
     const TileInfo& ti = kTileInfo[p.tile];
     const bool edges = ti.direct && (d->m % ti.bm != 0 || d->n % ti.bn != 0 || d->k % 16 != 0);
-    const KernelFn kernel = edges ? p.e->edge[has_bias][p.tile - kDirect] : p.e->k[has_bias][p.tile];
+    const bool few = d->kgroups == 1 && cdiv(cdiv(d->k, 16), p.splits) <= kFewChunks * (ti.bk / 16);
+    const KernelFn kernel = edges ? p.e->edge[few][has_bias][p.tile - kDirect] : p.e->k[has_bias][p.tile];
     PXK_LAUNCH(kernel, dim3(static_cast<unsigned>(blocks)), dim3(static_cast<unsigned>(ti.threads)), 0, S(stream), g);
     if (const int rc = launched("pxk_gemm")) return rc;
     if (p.splits > 1) {

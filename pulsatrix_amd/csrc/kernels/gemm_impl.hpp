@@ -81,6 +81,7 @@ struct Args {
 using KernelFn = void (*)(const Args);
 
 constexpr int kDirect = 4, kDirectTiles = 3;
+constexpr int kFewChunks = 3;  // chunks a wave that the direct tiles' short-K kernels hold in flight
 constexpr int kTiles = 10;  // gemm.hip's kPublicTile names them
 
 // One (transpose, prologue, epilogue) combination: its kernel on every tile shape, without and
@@ -89,7 +90,7 @@ struct Entry {
     int ta, tb, pro, epi;
     KernelFn k[2][kTiles];  // [prologue bias over k present][tile]
     KernelFn r[kTiles];
-    KernelFn edge[2][kDirectTiles];  // the direct tiles' kernels (from kDirect on) for ragged launches
+    KernelFn edge[2][2][kDirectTiles];  // the direct tiles' kernels (from kDirect on) for ragged launches: [few chunks][bias]
 };
 
 // The skinny kernels built: B layout, epilogue, kernels for up to 4, 8 and 16 rows (NN: with 64-,
@@ -954,12 +955,16 @@ struct DirectChunk {
     }
 };
 
-// EDGE: the launch has tiles that reach past M or N, or chunks past K. Without, none of their code is
-// in the kernel: these launches are short enough to feel their instruction fetches.
-template <class C, bool TA, bool TB, int PRO, int EPI, bool EDGE>
+// EDGES: the launch has tiles that reach past M or N, or chunks past K (kEdges), and no wave has more than
+// kFewChunks chunks, without k-groups (kEdgesFew). Each is a kernel of its own: these launches are short
+// enough to feel their instruction fetches.
+enum { kNoEdges, kEdges, kEdgesFew };
+template <class C, bool TA, bool TB, int PRO, int EPI, int EDGES>
 __global__ void __launch_bounds__(C::NT) gemm_direct_kernel(const Args g) {
     static_assert(C::WM == 1 && C::WN == 1, "direct loads: every wave owns the whole tile");
+    constexpr bool EDGE = EDGES != kNoEdges, FEW = EDGES == kEdgesFew;
     constexpr int BM = C::BM, BN = C::BN, TM = C::TM, TN = C::TN, KS = C::KS, PF = 3;
+    static_assert(PF == kFewChunks, "a short-K wave's chunks are in flight at once");
     __shared__ __attribute__((aligned(16))) float smem[KS * BM * C::LDC];
     __shared__ float s_rss[PRO == PXK_PRO_RMS ? KS * BM : 1];  // PXK_PRO_RMS: per K slice, each row's sum of squares
 
@@ -1017,27 +1022,23 @@ __global__ void __launch_bounds__(C::NT) gemm_direct_kernel(const Args g) {
         if (k_lo + 16 * static_cast<int64_t>(nch) > g.K && nw > 0)
             nf = g.kgroups != 1 ? 0 : (first + KS * (nw - 1) == nch - 1 ? nw - 1 : nw);
     }
-    // No more chunks than sets, and perhaps a ragged one: all are in flight at once. (The loop below would
-    // load its last chunk up to five times over and the ragged one after the others: 414 x 197 x 125 TN
+    // All of a short-K wave's chunks are in flight at once, a ragged one among them. (The loop below would
+    // load the last chunk up to five times over and the ragged one after the others: 414 x 197 x 125 TN
     // 5.8 us, 4.9 with every element guarded, 4.5 so; 5184 x 128 x 160 9.5, 9.0 and 8.2.)
-    bool rest = true;
-    if constexpr (EDGE) {
-        if (nf <= PF && (nf == nw || g.kgroups == 1)) {
-            DirectChunk<C, TA, TB, PRO> ch[PF], last;
-            static_for<PF>([&](auto U) {
-                if (U.value >= nf) return;
-                ch[U.value].template load<true>(g, A, Z, ZB, B, m0, n0, k_lo + 16 * kk, lane);
-                if (U.value + 1 < nf) advance();
-            });
-            if (nf < nw) last.load_guarded(g, A, Z, ZB, B, m0, n0, k_lo + 16 * static_cast<int64_t>(nch - 1), lane);
-            static_for<PF>([&](auto U) {
-                if (U.value < nf) ch[U.value].mma(acc, g.eps, ss);
-            });
-            if (nf < nw) last.mma(acc, g.eps, ss);
-            rest = false;
-        }
+    if constexpr (FEW) {
+        DirectChunk<C, TA, TB, PRO> ch[PF], last;
+        static_for<PF>([&](auto U) {
+            if (U.value >= nf) return;
+            ch[U.value].template load<true>(g, A, Z, ZB, B, m0, n0, k_lo + 16 * kk, lane);
+            if (U.value + 1 < nf) advance();
+        });
+        if (nf < nw) last.load_guarded(g, A, Z, ZB, B, m0, n0, k_lo + 16 * static_cast<int64_t>(nch - 1), lane);
+        static_for<PF>([&](auto U) {
+            if (U.value < nf) ch[U.value].mma(acc, g.eps, ss);
+        });
+        if (nf < nw) last.mma(acc, g.eps, ss);
     }
-    if (nf > 0 && rest) {
+    if (!FEW && nf > 0) {
         DirectChunk<C, TA, TB, PRO> ch[PF];
         auto load = [&](auto S) {  // the cursor's chunk -> set S; the cursor stops at the last one
             ch[S.value].template load<EDGE>(g, A, Z, ZB, B, m0, n0, k_lo + 16 * kk, lane);
@@ -1052,9 +1053,9 @@ __global__ void __launch_bounds__(C::NT) gemm_direct_kernel(const Args g) {
         }
         if (EDGE && nf < nw) advance();
     }
-    if constexpr (EDGE) {
+    if constexpr (EDGE && !FEW) {
         DirectChunk<C, TA, TB, PRO> ch;
-        for (int u = nf; u < nw && rest; ++u) {
+        for (int u = nf; u < nw; ++u) {
             ch.load_guarded(g, A, Z, ZB, B, m0, n0, k_lo + 16 * kk, lane);
             ch.mma(acc, g.eps, ss);
             if (u + 1 < nw) advance();
@@ -1753,13 +1754,16 @@ __global__ void __launch_bounds__(C::NT, 2) gemm_split_kernel(const Args g) {
 
 #define PXK_KSET(TA, TB, P, EPI)                                                                    \
     {gemm_kernel<C128, TA, TB, P, EPI>, gemm_kernel<C64, TA, TB, P, EPI>, gemm_kernel<C32x64, TA, TB, P, EPI>, \
-     gemm_kernel<C32, TA, TB, P, EPI>, gemm_direct_kernel<C32x64, TA, TB, P, EPI, false>,                  \
-     gemm_direct_kernel<C32, TA, TB, P, EPI, false>, gemm_direct_kernel<C32x48, TA, TB, P, EPI, false>,    \
+     gemm_kernel<C32, TA, TB, P, EPI>, gemm_direct_kernel<C32x64, TA, TB, P, EPI, kNoEdges>,                  \
+     gemm_direct_kernel<C32, TA, TB, P, EPI, kNoEdges>, gemm_direct_kernel<C32x48, TA, TB, P, EPI, kNoEdges>,    \
      gemm_kernel<C32x48, TA, TB, P, EPI>, gemm_split_kernel<S128, TA, TB, P, EPI>,                         \
      gemm_split_kernel<S64, TA, TB, P, EPI>}
-#define PXK_EDGES(TA, TB, P, EPI)                                                                         \
-    {gemm_direct_kernel<C32x64, TA, TB, P, EPI, true>, gemm_direct_kernel<C32, TA, TB, P, EPI, true>,     \
-     gemm_direct_kernel<C32x48, TA, TB, P, EPI, true>}
+#define PXK_EDGES(TA, TB, P, EPI, EDGES)                                                                  \
+    {gemm_direct_kernel<C32x64, TA, TB, P, EPI, EDGES>, gemm_direct_kernel<C32, TA, TB, P, EPI, EDGES>,   \
+     gemm_direct_kernel<C32x48, TA, TB, P, EPI, EDGES>}
+#define PXK_EDGES_BIAS(TA, TB, PRO, EPI, EDGES)                                                           \
+    {PXK_EDGES(TA, TB, PRO, EPI, EDGES),                                                                  \
+     PXK_EDGES(TA, TB, (PRO == PXK_PRO_DIV_STAB ? kProStabBias : PRO), EPI, EDGES)}
 #define PXK_GEMM_ENTRY(TA, TB, PRO, EPI)                                                                   \
     Entry {                                                                                                \
         TA, TB, PRO, EPI, {PXK_KSET(TA, TB, PRO, EPI), PXK_KSET(TA, TB, (PRO == PXK_PRO_DIV_STAB ? kProStabBias : PRO), EPI)}, \
@@ -1767,7 +1771,7 @@ __global__ void __launch_bounds__(C::NT, 2) gemm_split_kernel(const Args g) {
              splitk_reduce_kernel<32, EPI>, splitk_reduce_kernel<64, EPI>, splitk_reduce_kernel<32, EPI>,   \
              splitk_reduce_kernel<48, EPI>, splitk_reduce_kernel<48, EPI>,                                  \
              splitk_reduce_kernel<128, EPI>, splitk_reduce_kernel<64, EPI>},                                \
-            {PXK_EDGES(TA, TB, PRO, EPI), PXK_EDGES(TA, TB, (PRO == PXK_PRO_DIV_STAB ? kProStabBias : PRO), EPI)}, \
+            {PXK_EDGES_BIAS(TA, TB, PRO, EPI, kEdges), PXK_EDGES_BIAS(TA, TB, PRO, EPI, kEdgesFew)},        \
     }
 
 constexpr int skinny_rows(int mb) { return mb == 4 ? 16 : (mb == 8 ? 16 : 8); }
