@@ -23,6 +23,7 @@ int plan_tile(int id) {  // -1: none
 
 struct TileInfo {
     int bm, bn, bk, threads;
+    double start_us;  // a launch apart from its stages
     double floor_us;  // a K stage of a workgroup alone on its CU (load latency bound), measured
     double util;      // fp32 MFMA utilisation when several waves share a SIMD, measured (the split
                       // tiles' products run on the bf16 units: above 1)
@@ -30,21 +31,25 @@ struct TileInfo {
     bool whole;       // fast on whole tiles of aligned operands only (element-wise guards elsewhere)
 };
 
-// The split tiles' figures: 8192 x 2048 x 2048 gives 1.4 us per stage and workgroup of a CU for
+// The split tiles start 1.5 us later than the others (a longer prologue, epilogue and kernel). Over 4210
+// random products with K from 4 to 8192, planned with that (and the 32-row tiles' charge in estimate()) and
+// without: over 8% slower than the fp32 plan of the same shape 70 and 434 (4 x 4 x 4 with a prologue 4.6
+// us, 6.3 without; 1152 x 192 x 1856 TN 15.0 and 20.1), and 1.026 and 1.076 times the best plan measured.
+// Their other figures: 8192 x 2048 x 2048 gives 1.4 us per stage and workgroup of a CU for
 // 128x128 and 3072 x 3072 x 576 0.47 for 64x64 (0.54 at three to a CU: 512 x 576 x 3072 in 8 splits);
 // a lone workgroup (512 x 576 x 1536) 1.8 and 0.65.
 constexpr int kFp32Tiles = 8;
 const TileInfo kTileInfo[kTiles] = {
-    {128, 128, 32, C128::NT, 1.0, 0.75, false, true},
-    {64, 64, 32, C64::NT, 0.8, 0.65, false, true},
-    {32, 64, 64, C32x64::NT, 0.8, 0.55, false, true},
-    {32, 32, 64, C32::NT, 0.8, 0.5, false, true},
-    {32, 64, 64, C32x64::NT, 0.65, 0.55, true, false},
-    {32, 32, 64, C32::NT, 0.65, 0.5, true, false},
-    {32, 48, 64, C32x48::NT, 0.65, 0.55, true, false},
-    {32, 48, 64, C32x48::NT, 0.8, 0.55, false, true},
-    {128, 128, 32, S128::NT, 1.8, 1.18, false, false},
-    {64, 64, 32, S64::NT, 0.65, 0.79, false, false},
+    {128, 128, 32, C128::NT, 4.0, 1.0, 0.75, false, true},
+    {64, 64, 32, C64::NT, 4.0, 0.8, 0.65, false, true},
+    {32, 64, 64, C32x64::NT, 4.0, 0.8, 0.55, false, true},
+    {32, 32, 64, C32::NT, 4.0, 0.8, 0.5, false, true},
+    {32, 64, 64, C32x64::NT, 4.0, 0.65, 0.55, true, false},
+    {32, 32, 64, C32::NT, 4.0, 0.65, 0.5, true, false},
+    {32, 48, 64, C32x48::NT, 4.0, 0.65, 0.55, true, false},
+    {32, 48, 64, C32x48::NT, 4.0, 0.8, 0.55, false, true},
+    {128, 128, 32, S128::NT, 5.5, 1.8, 1.18, false, false},
+    {64, 64, 32, S64::NT, 5.5, 0.65, 0.79, false, false},
 };
 
 constexpr int kSkinnyMaxLds = 64 * 1024;
@@ -163,7 +168,10 @@ double estimate(const pxk_gemm_desc* d, const TileInfo& t, double tiles, double 
         util *= 0.75;
     }
     const double stage_us = std::max(floor, waves_per_simd * mfma_us / util);
-    double us = 4.0 + per * stage_us;
+    double us = t.start_us + per * stage_us;
+    // LDS-staged 32-row tiles, several to a CU, beside the split ones: 4352 x 640 x 64 17.2 us, 64x64 split
+    // 10.2, where their stages alone would tell 8.7 from 8.7.
+    if (!t.direct && t.bm == 32 && !d->denominator) us += 0.5 * std::max(0.0, waves_per_simd - 1.0);
     // The reduction launch (its own latency floor) and the partials' round trip through HBM. At
     // 512 x 576 x 3072 the unsplit direct tile beats split-K 4 with its reduce by about 1 us.
     if (splits > 1) us += 7.5 + 2.0 * splits * d->batch * d->m * d->n * 4.0 / 5.0e6;
