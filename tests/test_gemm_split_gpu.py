@@ -1,6 +1,7 @@
 """The split-bf16 GEMM tiles (128x128, 64x64) and the clamped edges of the direct ones, where they can
-go wrong: rows, columns and K past the tiles, short and ragged K, unaligned rows, split-K, and
-operands that the split itself does not settle (infinities, NaN, overflow, values near underflow).
+go wrong: rows, columns and K past the tiles, short and ragged K, unaligned rows, split-K, causal ranges,
+K-groups and batch strides, leading dimensions past 32-bit offsets, and operands that the split itself
+does not settle (infinities, NaN, overflow) or settles by its scale (values near underflow).
 
 The bound of the ordinary cases: each product of three-part operands is off by at most 2^-25 of its
 size, the accumulators add K / 32 roundings of 2^-24, and a 2-norm over normal operands averages them:
@@ -57,8 +58,8 @@ def test_edges_match_float64(tile, ta, tb, m, n, k, splits):
 @pytest.mark.parametrize("tile", TILES)
 @pytest.mark.parametrize("splits", [1, 2])
 def test_values_the_split_cannot_hold(tile, splits):
-    """Infinities, NaN, products that overflow and operands whose low bf16 parts underflow come out as the
-    fp32 tiles give them."""
+    """Infinities, NaN and products that overflow come out as the fp32 tiles give them, and small results to
+    their last bits."""
     rng = np.random.RandomState(7)
     a, b = rng.standard_normal((150, 200)).astype(np.float32), rng.standard_normal((200, 140)).astype(np.float32)
     a[3, 5], a[70, 9], a[100, 1] = np.inf, np.nan, 3.4e38
@@ -125,15 +126,108 @@ def test_rows_past_32_bit_offsets():
 
 @gpu
 @pytest.mark.parametrize("tile", TILES)
-def test_no_less_exact_than_the_fp32_tiles(tile):
-    """Against float64 on normal, positive and heavy-tailed operands, beside the fp32 MFMA's direct tile. The
-    split tiles stand where one fp32 accumulator ran over the whole of K; the direct tile adds four
-    quarters of it, with a quarter of the roundings each and so half the error: the bound is twice its."""
+@pytest.mark.parametrize("causal", [N.CAUSAL_NONE, N.CAUSAL_TRI, N.CAUSAL_K_LE_M, N.CAUSAL_K_GE_M])
+@pytest.mark.parametrize("kgroups,k", [(1, 256), (1, 201), (3, 64), (3, 75)])
+@pytest.mark.parametrize("splits", [1, 2])
+def test_causal_ranges_groups_and_strides(tile, causal, kgroups, k, splits):
+    """Batches of 2 x 2 with B shared by the inner two (a KV head), K-groups strided apart, and the causal
+    ranges, whose tiles neither read K outside their range (NaN here) nor compute above the diagonal."""
+    m, n = (k, 70) if causal in (N.CAUSAL_K_LE_M, N.CAUSAL_K_GE_M) else (201, 140)
+    rng = np.random.RandomState(k + causal)
+    a, b = rng.standard_normal((4, kgroups, m, k)).astype(np.float32), rng.standard_normal((2, kgroups, k, n)).astype(np.float32)
+    rows, cols, bm = np.arange(m)[:, None], np.arange(k)[None], 128 if tile == N.TILE_128x128_SPLIT else 64
+    if causal == N.CAUSAL_K_LE_M:
+        a[..., cols > rows] = 0.0
+        a[..., cols >= (rows // bm + 1) * bm] = np.nan
+    if causal == N.CAUSAL_K_GE_M:
+        a[..., cols < rows] = 0.0
+        a[..., cols < rows // bm * bm] = np.nan
+    want = np.einsum("bgmk,bgkn->bmn", np.nan_to_num(a).astype(np.float64), np.repeat(b, 2, axis=0).astype(np.float64))
+    da, db, dc = G.dev(a), G.dev(b), G.empty((4, m, n))
+    ws = G.empty((splits * 4 * m * n,))
+    d = N.GemmDesc()
+    d.m, d.n, d.k, d.batch, d.inner, d.kgroups, d.causal, d.tile, d.splits = m, n, k, 4, 2, kgroups, causal, tile, splits
+    d.a = N.operand(da.data_ptr(), k, 2 * kgroups * m * k, kgroups * m * k, 1, m * k)
+    d.b = N.operand(db.data_ptr(), n, kgroups * k * n, kgroups * k * n, 2, k * n)
+    d.c = N.operand(dc.data_ptr(), n, 2 * m * n, m * n, 1)
+    d.workspace, d.workspace_bytes = ws.data_ptr(), ws.numel() * 4
+    N.gemm(d, G.stream())
+    got = G.host(dc).reshape(4, m, n)
+    keep = np.tril(np.ones((m, n), bool)) if causal == N.CAUSAL_TRI else np.ones((m, n), bool)
+    assert np.linalg.norm((got - want)[:, keep]) <= 3e-7 * np.linalg.norm(want[:, keep])
+
+
+@gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_leading_dimensions_past_32_bit_offsets(tile, ta, tb):
+    """Rows 2^22 elements apart and further are loaded element by element."""
+    torch = G.torch_cuda()
+    m, n, k, ld = 70, 65, 40, (1 << 22) + 3
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    A, B = (torch.zeros(r, ld, device="cuda") for r in ((k if ta else m), (n if tb else k)))
+    a, b = A[:, :m if ta else k], B[:, :k if tb else n]
+    a.copy_(torch.randn(a.shape, device="cuda", generator=gen))
+    b.copy_(torch.randn(b.shape, device="cuda", generator=gen))
+    c = torch.empty(m, n, device="cuda")
+    d = N.GemmDesc()
+    d.m, d.n, d.k, d.batch, d.inner, d.kgroups, d.trans_a, d.trans_b, d.tile, d.splits = m, n, k, 1, 1, 1, ta, tb, tile, 1
+    d.a, d.b, d.c = N.operand(A.data_ptr(), ld), N.operand(B.data_ptr(), ld), N.operand(c.data_ptr(), n)
+    N.gemm(d, G.stream())
+    a, b = a.cpu().double().numpy(), b.cpu().double().numpy()
+    want = (a.T if ta else a) @ (b.T if tb else b)
+    assert np.linalg.norm(c.cpu().double().numpy() - want) <= 3e-7 * np.linalg.norm(want)
+    del A, B
+    torch.cuda.empty_cache()
+
+
+@gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("k", [96, 101])
+def test_values_the_split_cannot_hold_after_the_prologue(tile, bias, k):
+    """The divided operand with an infinity and a NaN, and quotients and products that overflow the split's
+    range: the tiles computed again divide too. Rows and columns without them stay exact."""
+    m, n, eps = 140, 70, 1e-6
+    rng = np.random.RandomState(k)
+    a, b = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    z = (rng.uniform(0.5, 1.5, (m, k)) * rng.choice([-1.0, 1.0], (m, k))).astype(np.float32)
+    zb = rng.uniform(-0.2, 0.2, k).astype(np.float32) if bias else np.zeros(k, np.float32)
+    x = rng.standard_normal((m, n)).astype(np.float32)
+    a[3, 5], a[70, 9], a[100, 1], a[139, k - 1] = np.inf, np.nan, 1e30, 1e32
+    zz = z.astype(np.float64) + zb
+    q = a / (zz + eps * np.where(zz >= 0, 1.0, -1.0))
+    with np.errstate(all="ignore"):
+        want = x * (q @ b.T.astype(np.float64))
+        scale = np.abs(x) * (np.abs(q) @ np.abs(b.T).astype(np.float64))
+    dc, keep = G.empty((m, n)), [G.dev(v) for v in (a, b, z, x, zb)]
+    d = N.GemmDesc()
+    d.m, d.n, d.k, d.batch, d.inner, d.kgroups, d.trans_b, d.tile, d.splits = m, n, k, 1, 1, 1, 1, tile, 1
+    d.prologue, d.epilogue, d.eps = N.PRO_DIV_STAB, N.EPI_MUL_X, eps
+    d.a, d.b, d.z, d.x = (N.operand(t.data_ptr(), w) for t, w in zip(keep, (k, k, k, n)))
+    if bias:
+        d.z_bias = N.operand(keep[4].data_ptr(), 0)
+    d.c = N.operand(dc.data_ptr(), n)
+    N.gemm(d, G.stream())
+    got = G.host(dc).reshape(m, n)
+    fine = np.isfinite(want)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
+    # a quotient takes a reciprocal within an ulp and two roundings, the products up to K / 4 more
+    assert np.all(np.abs(got - want)[fine] <= (4 + k / 4) * 2.0 ** -24 * scale[fine])
+
+
+@gpu
+@pytest.mark.parametrize("tile,fp32", [(N.TILE_128x128_SPLIT, N.TILE_128x128), (N.TILE_64x64_SPLIT, N.TILE_64x64)])
+@pytest.mark.parametrize("k", [64, 576, 1536, 8192])
+def test_no_less_exact_than_the_fp32_tiles(tile, fp32, k):
+    """Against float64 on normal, positive and heavy-tailed operands, beside the fp32 tile of the same size,
+    whose place each split tile takes."""
     rng = np.random.RandomState(3)
     for draw in (lambda *s: rng.standard_normal(s), lambda *s: np.abs(rng.standard_normal(s)),
                  lambda *s: rng.standard_normal(s) * np.exp(2.0 * rng.standard_normal(s))):
-        a, b = draw(96, 1536).astype(np.float32), draw(1536, 96).astype(np.float32)
+        a, b = draw(96, k).astype(np.float32), draw(k, 96).astype(np.float32)
         want = a.astype(np.float64) @ b.astype(np.float64)
-        err = [np.linalg.norm(product(a, b, 0, 0, t) - want) for t in (tile, N.TILE_32x32_DIRECT)]
-        print("split %.3g, fp32 in four K slices %.3g" % tuple(np.array(err) / np.linalg.norm(want)))
-        assert err[0] <= 2.0 * err[1]
+        err = [np.linalg.norm(product(a, b, 0, 0, t) - want) for t in (tile, fp32)]
+        print("split %.3g, fp32 %.3g" % tuple(np.array(err) / np.linalg.norm(want)))
+        assert err[0] <= err[1]

@@ -29,9 +29,13 @@ COMBOS = [
     (0, 1, N.PRO_NONE, N.EPI_SPV), (0, 1, N.PRO_NONE, N.EPI_SWIGLU_REL),
 ]
 TILES = [N.TILE_128x128, N.TILE_64x64, N.TILE_32x64, N.TILE_32x32, N.TILE_32x64_DIRECT, N.TILE_32x32_DIRECT,
-         N.TILE_32x48_DIRECT, N.TILE_32x48]
+         N.TILE_32x48_DIRECT, N.TILE_32x48, N.TILE_128x128_SPLIT, N.TILE_64x64_SPLIT]
 TILE_BN = {N.TILE_128x128: 128, N.TILE_64x64: 64, N.TILE_32x64: 64, N.TILE_32x32: 32, N.TILE_32x64_DIRECT: 64,
-           N.TILE_32x32_DIRECT: 32, N.TILE_32x48_DIRECT: 48, N.TILE_32x48: 48}
+           N.TILE_32x32_DIRECT: 32, N.TILE_32x48_DIRECT: 48, N.TILE_32x48: 48, N.TILE_128x128_SPLIT: 128,
+           N.TILE_64x64_SPLIT: 64}
+# Ragged M and K with few and with more 16-deep chunks a wave (the direct tiles' two kernels with edges),
+# and whole direct tiles and chunks (their third); N = whole heads for the RoPE rule.
+SHAPES = [(77, 128, 150), (77, 128, 230), (96, 192, 160)]
 EPS = 1e-6
 
 
@@ -130,14 +134,15 @@ def run(d, splits):
 
 
 @gpu
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "%dx%dx%d" % s)
 @pytest.mark.parametrize("splits", [1, 3])
 @pytest.mark.parametrize("tile", TILES)
 @pytest.mark.parametrize("combo", COMBOS, ids=lambda c: "ta%d_tb%d_pro%d_epi%d" % c)
-def test_fused_gemm_on_every_tile(combo, tile, splits):
+def test_fused_gemm_on_every_tile(combo, tile, splits, shape):
     ta, tb, pro, epi = combo
     rope = epi in (N.EPI_ROPE_REL, N.EPI_ROPE_FWD)
     D = 64 if rope and TILE_BN[tile] >= 64 else 16
-    m, n, k = 77, 128, 150  # ragged M and K; N = whole heads for the RoPE rule
+    m, n, k = shape
     a, b = G.uniform((k, m) if ta else (m, k), 1), G.uniform((n, k) if tb else (k, n), 2)
     t = {"x": G.uniform((m, n), 3), "y": away((m, n), 4), "w": away((m, n), 5), "z": away((m, n), 6),
          "z2": away((m, n), 7), "z3": away((m, n), 8), "c0": G.uniform((m, n), 9),
