@@ -182,11 +182,11 @@ typedef struct pxk_gemm_desc {
     const float* x_gamma;
     float* row_rms;          /* PXK_PRO_RMS: receives rms[m] (nullable) */
     float norm_eps;          /* PXK_PRO_RMS */
-    int32_t denominator;     /* 1: the product is, or feeds, a denominator of the epsilon rules (a forward
-                                pass kept for a relevance pass): PXK_TILE_AUTO then plans over the fp32
-                                tiles alone, whose rounding those rules' results have always had. Near a
-                                zero denominator eps / z turns a last-bit difference of z into one of the
-                                relevance, whichever of two equally exact products z came from. */
+    int32_t denominator;     /* 1: PXK_TILE_AUTO plans over the fp32 tiles alone. For a forward product kept
+                                for a relevance pass: near a zero denominator eps / z turns a last-bit
+                                difference of z into one of the relevance, and so these products' results
+                                keep the bits that the fp32 tiles give them. It is no matter of accuracy (the
+                                split tiles' z is the closer one), and a caller may leave it 0. */
 } pxk_gemm_desc;
 
 /* Bytes of workspace pxk_gemm needs for this descriptor (0 when it runs without split-K). */

@@ -67,7 +67,9 @@ inline pxk_gemm_desc gemm_desc(int64_t m, int64_t n, int64_t k) {
     d.batch = d.inner = d.kgroups = 1;
     return d;
 }
-/** @brief gemm_desc for a forward product that is, or feeds, a denominator of the relevance pass. */
+/** @brief gemm_desc for a layer's forward product, which is, or feeds, a denominator of its epsilon rule:
+ *         its bits stay those of the fp32 tiles. The tied head's logits and the affine rules' denominators
+ *         are planned freely (modules.cpp, rules.cpp). */
 inline pxk_gemm_desc forward_desc(int64_t m, int64_t n, int64_t k) {
     pxk_gemm_desc d = gemm_desc(m, n, k);
     d.denominator = 1;

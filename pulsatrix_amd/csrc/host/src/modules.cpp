@@ -310,6 +310,11 @@ const float* TiedLMHeadModule::run_forward(const float* x, int64_t rows) {
     x_ = x;
     rows_ = rows;
     float* logits = logits_.ensure(be_, rows * V);
+    // Planned freely (split tiles), though the logits are the head's epsilon denominators. A seeded pass
+    // divides by its target's logit alone; for a relevance of every entry, measured against float64 with
+    // logits from the fp32 and from the split tiles (24 seeds each of 512 x 49152 x 576, 203 x 49152 x 576 and
+    // 128 x 32000 x 2048, eps 1e-9 and 1e-6): logits off by 4.3e-7 and 1.4e-7 (8.1e-7 and 1.9e-7 at 2048),
+    // the relevance closer on the split tiles in 125 of 144, its median error 2 to 19 times smaller.
     pxk_gemm_desc d = gemm_desc(rows, V, D);
     d.trans_b = 1;  // E (V, D) read transposed in place
     d.a = mat(x, D);

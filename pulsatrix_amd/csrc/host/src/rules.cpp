@@ -79,7 +79,9 @@ void AffineRule::run(MI355XBackend* be, const LRPRuleConfig& config, uint64_t ve
     const int64_t wo = zbox ? out : 2 * out;  // W2's width: the GEMMs' output (den) or reduction (C) extent
     float* g = den_.ensure(be, rows * wo);
     if (!zbox) {
-        // den = [x+ | x-] W2: both stabilised denominators of every output in one GEMM.
+        // den = [x+ | x-] W2: both stabilised denominators of every output in one GEMM. Planned freely: the
+        // AlphaBeta sums hold terms of one sign, and a Gamma denominator is used where z has its sign, at
+        // least gamma times that sign's terms away from zero, so neither magnifies a last bit.
         float* xs = xs_.ensure(be, rows * 2 * in);
         MI355XBackend::check(pxk_lrp_sign_split(p.x, p.ldx, rows, in, xs, st), "lrp rule sign split");
         pxk_gemm_desc d = gemm_desc(rows, wo, 2 * in);
