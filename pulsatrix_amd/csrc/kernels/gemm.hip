@@ -33,7 +33,7 @@ struct TileInfo {
 
 // The split tiles start 1.5 us later than the others (a longer prologue, epilogue and kernel). Over 4210
 // random products with K from 4 to 8192, planned with that (and the 32-row tiles' charge in estimate()) and
-// without: over 8% slower than the fp32 plan of the same shape 70 and 434 (4 x 4 x 4 with a prologue 4.6
+// without: over 8% slower than the fp32 plan of the same shape 69 and 434 (4 x 4 x 4 with a prologue 4.6
 // us, 6.3 without; 1152 x 192 x 1856 TN 15.0 and 20.1), and 1.026 and 1.076 times the best plan measured.
 // Their other figures: 8192 x 2048 x 2048 gives 1.4 us per stage and workgroup of a CU for
 // 128x128 and 3072 x 3072 x 576 0.47 for 64x64 (0.54 at three to a CU: 512 x 576 x 3072 in 8 splits);
@@ -169,9 +169,9 @@ double estimate(const pxk_gemm_desc* d, const TileInfo& t, double tiles, double 
     }
     const double stage_us = std::max(floor, waves_per_simd * mfma_us / util);
     double us = t.start_us + per * stage_us;
-    // LDS-staged 32-row tiles, several to a CU, beside the split ones: 4352 x 640 x 64 17.2 us, 64x64 split
-    // 10.2, where their stages alone would tell 8.7 from 8.7.
-    if (!t.direct && t.bm == 32 && !d->denominator) us += 0.5 * std::max(0.0, waves_per_simd - 1.0);
+    // LDS-staged 32-row tiles in one pass, several to a CU, beside the split ones: 4352 x 640 x 64 17.2 us,
+    // 64x64 split 10.2, where their stages alone would tell 8.7 from 8.7.
+    if (!t.direct && t.bm == 32 && splits == 1 && !d->denominator) us += 0.5 * std::max(0.0, waves_per_simd - 1.0);
     // The reduction launch (its own latency floor) and the partials' round trip through HBM. At
     // 512 x 576 x 3072 the unsplit direct tile beats split-K 4 with its reduce by about 1 us.
     if (splits > 1) us += 7.5 + 2.0 * splits * d->batch * d->m * d->n * 4.0 / 5.0e6;
