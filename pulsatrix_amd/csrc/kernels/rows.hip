@@ -41,7 +41,8 @@ __global__ void __launch_bounds__(kThreads) rms_norm_kernel(const float* in, con
 // owns float4 columns l, l + 64, ..., so x is read from HBM once. Needs cols % 4 == 0, 16-byte
 // aligned rows, and cols <= 256 * NV. NT: streaming (non-temporal) cache policy for x and out, for
 // tensors far larger than the caches. Otherwise, up to 1024 columns, gamma is read with x and not after
-// the reduction: a decode step's one row is the latency of its loads (1 x 576: 4.1 -> 3.5 us).
+// the reduction: a decode step's one row is the latency of its loads (1 x 576 among a decode step's other
+// launches 4.13 -> 3.83 us, a 200-token prompt and 16 steps of 30 layers 28.8 -> 27.5 ms).
 template <int NV, bool NT>
 __global__ void __launch_bounds__(kThreads) rms_norm_vec_kernel(const float* in, const float* gamma, float* out,
                                                                 float* row_rms, int64_t rows, int cols4, float eps) {
@@ -131,7 +132,8 @@ struct NormAddArgs {
 //
 // A decode step runs this on a row or a few, where the launch is the memory latency of its loads one
 // after the other: up to 1024 columns (NV <= 4) x and both gammas are therefore read with a, before
-// the first reduction. Wider rows keep them behind it, for the registers. 4 x 640: 6.3 -> 4.3 us.
+// the first reduction. Wider rows keep them behind it, for the registers. 4 x 640 among a decode step's
+// other launches: 6.3 -> 4.3 us.
 template <int NV>
 __global__ void __launch_bounds__(kThreads) rms_norm_add_vec_kernel(const NormAddArgs g) {
     typedef float f4 __attribute__((ext_vector_type(4)));
