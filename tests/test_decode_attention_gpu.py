@@ -64,3 +64,11 @@ def test_chunks_of_scores_minus_infinity(cap, pos, masked, D):
 @pytest.mark.parametrize("D", [64, 320])
 def test_long_caches(cap, pos, D):
     run(1, 2, 1, D, cap, pos, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [132, 256])
+@pytest.mark.parametrize("n,cap", [(1, 4096), (1, 4097), (4, 1088)])
+def test_wide_heads_in_small_and_large_grids(n, cap, D):
+    """Head_dims past 128 on both sides of the 512 workgroups up to which a chunk is held in registers."""
+    run(n, 8, 2, D, cap, cap - 1, 0)

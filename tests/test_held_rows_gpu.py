@@ -10,8 +10,8 @@ import pytest
 import gpu_util as G
 from pulsatrix_amd import native as N
 
-COLS = [1, 3, 63, 64, 65, 255, 256, 257, 260, 508, 512, 516, 1023, 1024, 1025, 1028, 2047, 2048, 2049, 2052, 4096, 4100, 8191, 8192, 8193,
-        8196]
+COLS = [1, 3, 63, 64, 65, 127, 128, 129, 132, 255, 256, 257, 260, 508, 511, 512, 513, 516, 1023, 1024, 1025, 1028, 1535, 1536, 1537, 2047,
+        2048, 2049, 2052, 3071, 3073, 4095, 4096, 4097, 4100, 6143, 6145, 8191, 8192, 8193, 8196]
 
 
 def _call(name, *args):
