@@ -327,27 +327,32 @@ __global__ void __launch_bounds__(kThreads) decode_attention_merge_few_kernel(co
     float ahead[kAhead];
 #pragma unroll
     for (int c = 0; c < kAhead; ++c) ahead[c] = col[min(c, nc - 1) * ps];
+    // A chunk without keys has a weight of 0 and a partial of zeros; one with keys whose maximum is -inf (NaN
+    // partials) is left out of the sums, which then select.
+    bool masked = false;
     if (tid < kWave) {
         const float m = tid < nc ? part[tid * ps] : -INFINITY;
         mass[tid] = tid < nc ? part[tid * ps + 1] : 0.0f;
         const float M = wave_max(m);
-        weight[tid] = m != -INFINITY ? expf(m - M) : -1.0f;  // -1: counts for nothing
+        masked = m == -INFINITY && mass[tid] != 0.0f;
+        weight[tid] = masked ? -1.0f : m != -INFINITY ? expf(m - M) : 0.0f;
     }
-    __syncthreads();
-    auto weighed = [&](int c, float x) {  // selects, no branches: the loads below issue back to back
-        const float w = weight[c];
-        return w < 0.0f ? 0.0f : w * x;
-    };
-    float l = 0.0f;
-    for (int c = 0; c < nc; ++c) l += weighed(c, mass[c]);
-    for (int64_t d = tid; d < a.D; d += kThreads) {
-        float acc = 0.0f;
+    auto sums = [&](auto weighed) {
+        float l = 0.0f;
+        for (int c = 0; c < nc; ++c) l += weighed(c, mass[c]);
+        for (int64_t d = tid; d < a.D; d += kThreads) {
+            float acc = 0.0f;
 #pragma unroll
-        for (int c = 0; c < kAhead; ++c)
-            if (c < nc) acc += weighed(c, d == tid ? ahead[c] : part[c * ps + kPartHead + d]);
-        for (int c = kAhead; c < nc; ++c) acc += weighed(c, part[c * ps + kPartHead + d]);
-        a.ctx[bh * a.D + d] = acc / l;
-    }
+            for (int c = 0; c < kAhead; ++c)
+                if (c < nc) acc += weighed(c, d == tid ? ahead[c] : part[c * ps + kPartHead + d]);
+            for (int c = kAhead; c < nc; ++c) acc += weighed(c, part[c * ps + kPartHead + d]);
+            a.ctx[bh * a.D + d] = acc / l;
+        }
+    };
+    if (__syncthreads_or(masked))
+        sums([&](int c, float x) { return weight[c] < 0.0f ? 0.0f : weight[c] * x; });
+    else
+        sums([&](int c, float x) { return weight[c] * x; });
 }
 
 __global__ void __launch_bounds__(kThreads) decode_attention_merge_kernel(const DecodeAttnArgs a) {
